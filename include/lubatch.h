@@ -145,7 +145,8 @@ int lu_ragged_invalid_count(const lub_ragged_plan* plan, int* out);
  * Per-n launch choices used when flags carry LUB_LAYOUT_AUTO: layout[n]
  * (0 = 16-lane rows, 1 = quads; quads apply to n <= 16 in the plain kernel,
  * n <= 12 in the ragged one) and grab[n] (ragged: wave tiles per work item,
- * >= 1, used up to 16 matrices per item).  Arrays of 33 entries indexed by n
+ * >= 1, used up to 64 matrices per item and less in batches too small to
+ * fill the GPU that way).  Arrays of 33 entries indexed by n
  * (entry 0 unused). */
 int lu_tuning_set(const signed char* layout, const signed char* grab);
 int lu_tuning_get(signed char* layout, signed char* grab);

@@ -18,7 +18,8 @@
 //             0 publishes it) -- size classes ordered largest n first; per
 //             class its first slot, its first descriptor, its lane layout and
 //             the matrices per descriptor (MPW(n) * grab(n) <= 64: MPW is 4
-//             with 16-lane rows, 16 with quads) -- then writes each matrix's
+//             with 16-lane rows, 16 with quads; grab is bounded by the batch's
+//             tile count, ragged_grab_limit) -- then writes each matrix's
 //             offset and pivot offset to its slot (class first + the block's
 //             first slot + a rank from an LDS atomic), so a descriptor's
 //             matrices sit in consecutive slots
@@ -31,6 +32,9 @@
 //             routines; each matrix is gathered and scattered by its own lane
 //             group, and the loads of tile b+1 are issued before the stores
 //             of tile b.
+//
+// Batches of up to 2,048 matrices are inverted without a plan, one wave per
+// matrix (lu_ragged_kernel's direct form).
 //
 // A matrix's result does not depend on which tile or slot it lands in: every
 // tile routine treats its matrices independently (the serial fallback of the
@@ -72,6 +76,23 @@ struct RaggedWs {
 
 constexpr int kRaggedQuadMaxN = 12;
 constexpr int kRaggedMaxPer = 64;  // matrices per descriptor: one slot per lane
+
+// The tuned grab amortises a descriptor's start-up where the chip is full;
+// in a small batch it would only chain tiles in one wave while compute units
+// idle.  So a descriptor takes no more than 1 / kRaggedTilesPerGrab of the
+// batch's tiles.  Mixed n = 4..32, us for grab 1 / 2 / 4 / 8 / the table (8,
+// 4 and 16): 3,000 matrices 20 / 28 / 44 / 77 / 131; 32,768 50 / 50 / 58 / 89
+// / 145; 100,000 (19k tiles) 113 / 109 / 115 / 123 / 175.  From 64k tiles
+// (about 350,000 such matrices) the table's 8 stands.
+constexpr int kRaggedTilesPerGrab = 8192;
+__host__ __device__ constexpr int64_t ragged_grab_limit(int64_t tiles) {
+  return tiles / kRaggedTilesPerGrab > 1 ? tiles / kRaggedTilesPerGrab : 1;
+}
+
+// Batches of up to kRaggedDirectMax matrices skip the plan: each matrix gets
+// a wave of its own (a 16-lane row of it), all resident at once (8 waves per
+// CU).  256 matrices: 12.6 us against 15.6 with the plan, 1,000: 13.1 / 16.7.
+constexpr int64_t kRaggedDirectMax = 2048;
 
 __host__ __device__ constexpr int ragged_mpw(int n, int layout) { return (layout == 1 && n <= kRaggedQuadMaxN) ? 16 : 4; }
 
@@ -281,7 +302,7 @@ struct RaggedDesc {
   int n;
   int layout;  // 0: 16-lane rows, 1: quads
   int first;   // first slot
-  int count;   // matrices (<= 16)
+  int count;   // matrices (<= kRaggedMaxPer)
 };
 
 // Class table of the plan, lane c (1..32) holding class c.
@@ -355,16 +376,36 @@ __device__ __forceinline__ void ragged_dispatch(const RaggedDesc& d, const Ragge
 // least the descriptor count each workgroup does one descriptor and the
 // hardware dispatcher starts a new wave whenever one ends; a resident-size
 // grid makes the waves persistent.
+// With `direct_ns` (the batch's own size array; soffs and spoffs are then its
+// offset arrays) there is no plan: descriptor t is matrix t alone, and
+// descriptor `batch` counts the matrices with n outside 1..32.
 template <int PIV>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void lu_ragged_kernel(
     float* __restrict__ A, const int64_t* __restrict__ soffs, int* __restrict__ piv,
-    const int64_t* __restrict__ spoffs, const int* __restrict__ hdr) {
+    const int64_t* __restrict__ spoffs, int* __restrict__ hdr, const int* __restrict__ direct_ns, int batch,
+    int direct_layout) {
   __shared__ __attribute__((aligned(16))) float lds[kRaggedLdsFloats];
   const int lane = threadIdx.x;
-  const RaggedClasses cls = ragged_load_classes(hdr, lane);
-  const int total = __builtin_amdgcn_readlane(cls.desc_first, 0);
+  RaggedClasses cls{};
+  int total = batch + 1;
+  if (direct_ns == nullptr) {
+    cls = ragged_load_classes(hdr, lane);
+    total = __builtin_amdgcn_readlane(cls.desc_first, 0);
+  }
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
-    const RaggedDesc d = ragged_locate(cls, t, lane);
+    RaggedDesc d;
+    if (direct_ns == nullptr) {
+      d = ragged_locate(cls, t, lane);
+    } else if (t < batch) {
+      d = RaggedDesc{__builtin_amdgcn_readfirstlane(direct_ns[t]), direct_layout, t, 1};
+      if (d.n < 1 || d.n > 32) continue;
+    } else {
+      int bad = 0;
+      for (int i = lane; i < batch; i += kWave) bad += (direct_ns[i] < 1 || direct_ns[i] > 32) ? 1 : 0;
+      for (int s = kWave / 2; s > 0; s >>= 1) bad += __shfl_xor(bad, s);
+      if (lane == 0) hdr[RaggedWs::META + 2] = bad;
+      continue;
+    }
     const RaggedSlots sl = ragged_load_slots(soffs, spoffs, d, lane);
     // Opaque per descriptor: keeps the lane-derived addresses of all the
     // (n, layout) variants from being hoisted out of the loop, where they

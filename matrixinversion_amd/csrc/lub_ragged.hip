@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_scan(int* __restrict__ ws
 // The class table from the class totals: classes 32, 31, ..., 1 in order;
 // a descriptor holds MPW(n) * grab(n) matrices, at most kRaggedMaxPer (one
 // slot per lane), so grab is clamped to 16 with 16-lane rows and 4 with
-// quads.  Every scatter block derives it (32 values); block 0 publishes it
+// quads, and to ragged_grab_limit of the batch's tiles.  Every scatter block derives it (32 values); block 0 publishes it
 // in the header for the inversion kernel.
 __device__ void ragged_class_table(int* __restrict__ ws, int64_t batch, const RaggedTuning& tune, bool publish,
                                    int* first_slot) {
@@ -121,14 +121,20 @@ __device__ void ragged_class_table(int* __restrict__ ws, int64_t batch, const Ra
   __shared__ int tiles_of[33];
   __shared__ int lper[33];
   const int c = threadIdx.x;
-  if (c >= 1 && c <= 32) {
-    const int cnt = ws[RaggedWs::COUNTS + c];
-    const int layout = (tune.layout[c] == 1 && c <= kRaggedQuadMaxN) ? 1 : 0;
+  if (c < kWave) {  // the first wave, whole: its lanes add up the tiles
+    const bool row = c >= 1 && c <= 32;
+    const int cnt = row ? ws[RaggedWs::COUNTS + c] : 0;
+    const int layout = (row && tune.layout[c] == 1 && c <= kRaggedQuadMaxN) ? 1 : 0;
     const int mpw = ragged_mpw(c, layout);
-    const int per_desc = mpw * min(max(1, (int)tune.grab[c]), kRaggedMaxPer / mpw);
-    count[c] = cnt;
-    tiles_of[c] = (cnt + per_desc - 1) / per_desc;
-    lper[c] = layout | (per_desc << 8);
+    int tiles = (cnt + mpw - 1) / mpw;
+    for (int s = kWave / 2; s > 0; s >>= 1) tiles += __shfl_xor(tiles, s);
+    if (row) {
+      const int grab = min(max(1, (int)tune.grab[c]), (int)ragged_grab_limit(tiles));
+      const int per_desc = mpw * min(grab, kRaggedMaxPer / mpw);
+      count[c] = cnt;
+      tiles_of[c] = (cnt + per_desc - 1) / per_desc;
+      lper[c] = layout | (per_desc << 8);
+    }
   }
   __syncthreads();
   if (c == 0) {
@@ -270,9 +276,16 @@ int64_t ragged_grid(int cus, const lub::RaggedTuning& rt, int64_t batch) {
     return e != nullptr ? std::atoi(e) : 0;
   }();
   if (per_cu > 0 && cus > 0) return int64_t(cus) * per_cu;
-  int min_per = lub::kRaggedMaxPer;
-  for (int n = 1; n <= 32; ++n) min_per = std::min(min_per, ragged_per(rt, n));
-  return std::min<int64_t>((batch + min_per - 1) / min_per + 32, int64_t(1) << 25);  // grid * 64 within 32 bits
+  int min_per = lub::kRaggedMaxPer, min_mpw = lub::kRaggedMaxPer;
+  for (int n = 1; n <= 32; ++n) {
+    min_per = std::min(min_per, ragged_per(rt, n));
+    min_mpw = std::min(min_mpw, lub::ragged_mpw(n, rt.layout[n]));
+  }
+  // Where ragged_grab_limit binds, a descriptor has at least half of
+  // tiles / kRaggedTilesPerGrab tiles (or one), plus one partial per class.
+  const int64_t tuned = (batch + min_per - 1) / min_per;
+  const int64_t bound = std::min<int64_t>((batch + min_mpw - 1) / min_mpw, 2 * int64_t(lub::kRaggedTilesPerGrab));
+  return std::min<int64_t>(std::max(tuned, bound) + 64, int64_t(1) << 25);  // grid * 64 within 32 bits
 }
 
 int check_ragged_args(float* A, const int64_t* offsets, const int* ns, int* piv, const int64_t* piv_offsets,
@@ -309,6 +322,17 @@ int enqueue_ragged(char* ws, int64_t capacity, int cus, float* A, const int64_t*
   int* bhist = reinterpret_cast<int*>(ws + lub::RaggedWs::bhist_offset());
   int64_t* soffs = reinterpret_cast<int64_t*>(ws + lub::RaggedWs::slots_offset(capacity));
   int64_t* spoffs_all = soffs + capacity;
+  const int* direct_ns = nullptr;
+  int count = static_cast<int>(batch);
+  int direct_layout = (flags & LUB_LAYOUT_MASK) == LUB_LAYOUT_QUAD4 ? 1 : 0;
+  if (batch <= lub::kRaggedDirectMax) {
+    const int64_t* no_plan_offs = offsets;
+    const int64_t* no_plan_poffs = piv ? piv_offsets : nullptr;
+    direct_ns = ns;
+    void* args[] = {&A, &no_plan_offs, &piv, &no_plan_poffs, &hdr, &direct_ns, &count, &direct_layout};
+    const hipError_t e = hipLaunchKernel(fn, dim3(static_cast<unsigned>(batch + 1)), dim3(64), args, 0, s);
+    return e == hipSuccess ? LUB_OK : LUB_EHIP;
+  }
   if (batch <= lub::kSmallPlanMax) {
     lub::ragged_plan_small<<<1, lub::kSmallPlanThreads, 0, s>>>(ns, offsets, piv ? piv_offsets : nullptr, batch, hdr,
                                                                 rt, soffs, spoffs_all);
@@ -321,8 +345,7 @@ int enqueue_ragged(char* ws, int64_t capacity, int cus, float* A, const int64_t*
                                                               bhist, nblocks, rt, soffs, spoffs_all);
   }
   int64_t* spoffs = piv ? spoffs_all : nullptr;
-  const int* hdr_arg = hdr;
-  void* args[] = {&A, &soffs, &piv, &spoffs, &hdr_arg};
+  void* args[] = {&A, &soffs, &piv, &spoffs, &hdr, &direct_ns, &count, &direct_layout};
   const int64_t grid = ragged_grid(cus, rt, batch);
   hipError_t e = hipLaunchKernel(fn, dim3(static_cast<unsigned>(grid)), dim3(64), args, 0, s);
   if (e != hipSuccess) return LUB_EHIP;

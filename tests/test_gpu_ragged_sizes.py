@@ -1,0 +1,69 @@
+"""Ragged batches on both sides of every size rule: no plan up to 2,048
+matrices, the one-workgroup plan up to 16,384, the three-step plan above, and
+the work items' tile count, which grows with the batch.  Every matrix must
+equal its plain launch bit for bit, and matrices of invalid n stay untouched
+and are counted."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+PER_N = 5  # distinct matrices of each n
+
+
+@pytest.fixture(scope="module")
+def pools(gpu):
+    """rule -> [n] (matrices, plain inverses, plain pivots)"""
+    out = {}
+    for name, flags in (("parallel", 0x1), ("none", 0x0), ("tree", 0x3), ("gepp", 0x4)):
+        out[name] = [None]
+        for n in range(1, 33):
+            gen = oracle.dominant_matrices if name == "none" else oracle.uniform_matrices
+            a = gen(900 + n, PER_N, n)
+            out[name].append((a, *gpu.invert(a, flags)))
+    return out
+
+
+@pytest.mark.parametrize("mode,flags", [("parallel", 0x1), ("none", 0x0), ("tree", 0x3), ("gepp", 0x4),
+                                        ("parallel", 0x11), ("parallel", 0x21)])
+@pytest.mark.parametrize("batch", [1, 7, 2047, 2048, 2049, 16384, 16385, 60001])
+def test_every_plan_rule_matches_plain(gpu, pools, mode, flags, batch):
+    rng = np.random.RandomState(batch + flags)
+    pool = pools[mode]
+    ns = rng.randint(1, 33, batch).astype(np.int32)
+    pick = rng.randint(0, PER_N, batch)
+    bad = rng.permutation(batch)[:batch // 50]
+    gaps = rng.randint(0, 3, batch)
+    offs = np.cumsum(gaps + ns.astype(np.int64) ** 2) - ns.astype(np.int64) ** 2
+    poffs = np.cumsum(ns.astype(np.int64)) - ns
+    total, ptotal = int(offs[-1]) + int(ns[-1]) ** 2 + 3, int(ns.sum())
+    flat = np.full(total, np.float32(-7.25), np.float32)
+    want, pwant = flat.copy(), np.full(ptotal, -1, np.int32)
+    given = ns.copy()
+    given[bad] = rng.choice([0, -3, 33, 1000], bad.size)
+    for i, (n, k) in enumerate(zip(ns, pick)):
+        o, po = offs[i], poffs[i]
+        a, x, p = pool[n]
+        flat[o:o + n * n] = a[k].ravel()
+        skipped = given[i] != n
+        want[o:o + n * n] = (a if skipped else x)[k].ravel()
+        if not skipped:
+            pwant[po:po + n] = p[k]
+    A, O, NS, PO = (gpu.DeviceBuffer.from_array(v) for v in (flat, offs, given, poffs))
+    P = gpu.DeviceBuffer.from_array(np.full(ptotal, -1, np.int32))
+    plan = gpu.RaggedPlan(batch)
+    try:
+        print(f"[case] ragged mode={mode} flags={flags:#x} batch={batch}", flush=True)
+        gpu.lu_batched_inverse_ragged(A, O, NS, batch, flags, P, PO, plan=plan)
+        gpu.synchronize()
+        x, p = A.download(flat.shape, np.float32), P.download((ptotal,), np.int32)
+        count = plan.invalid_count()
+    finally:
+        plan.close()
+        for b in (A, O, NS, PO, P):
+            b.close()
+    assert np.array_equal(x.view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(p, pwant)
+    assert count == bad.size
