@@ -8,18 +8,21 @@
 // its inverse is the FP32 LU result (parallel_pivot/luBatchedInplace.cuh:
 // 84-125, stored at :194-197).
 //
-// Per tile of four matrices (one wave, 16 lanes per matrix, n = 17..32):
+// Per tile (one wave; 16 lanes per matrix and 4 matrices for n > 12, quads
+// and 16 matrices up to n = 12, as in the plain kernel):
 //   1. the tile arrives in registers (TileRegs) and is staged into LDS;
-//   2. tile_front + tile_solve leave X = A^-1 in the tile's LDS region;
-//   3. per matrix, the whole wave: A_m is read a second time (normally from
-//      the caches) straight into the FP64 product's operand registers,
-//      D = A_m X_m is formed on the FP64 matrix cores (v_mfma_f64_16x16x4f64:
-//      products of FP32 values are exact in FP64, the sums round in FP64),
-//      E = D - I (= -R) is rounded to FP32 and stays in the registers it was
-//      accumulated in, which are exactly the operands of C = X_m E on the
-//      FP32 matrix cores (v_mfma_f32_16x16x4f32, accumulated from zero so its
-//      roundings stay at the correction's scale), and X_m - C (one rounding)
-//      replaces X_m in LDS;
+//   2. tile_front + tile_solve (tile_gepp) leave X = A^-1 in the tile's LDS
+//      region; the form that refines a given X (kPivGiven) stages X instead;
+//   3. per matrix (per 2 or 4 matrices up to n = 8 or 4), the whole wave: A_m
+//      is read a second time (normally from the caches) straight into the
+//      FP64 product's operand registers, D = A_m X_m is formed on the FP64
+//      matrix cores (v_mfma_f64_16x16x4f64: products of FP32 values are exact
+//      in FP64, the sums round in FP64), E = D - I (= -R) is rounded to FP32
+//      and stays in the registers it was accumulated in, which are exactly
+//      the operands of C = X_m E on the FP32 matrix cores
+//      (v_mfma_f32_16x16x4f32, accumulated from zero so its roundings stay at
+//      the correction's scale), and X_m - C (one rounding) replaces X_m in
+//      LDS;
 //   4. the tile goes to HBM with the plain kernel's coalesced tile store.
 // Nothing but the tile itself lives in LDS, so the kernel keeps the plain
 // kernel's occupancy.  Padding: A_m's registers hold zeros outside its n x n
@@ -186,80 +189,205 @@ __device__ __forceinline__ void refined_step(const RefinedA& am, float* xm, int 
       }
 }
 
-// Out-of-place inverse + one refinement step of `batch` n x n matrices
-// (n = 17..32, 16 lanes per matrix): A is only read, X receives the refined
-// inverse, piv (nullable) the pivot vectors.  `vec`: bit 0, A is 16-byte
-// aligned; bit 1, X is.  One workgroup (one wave) per tile of four matrices,
-// striding when the grid is capped; a striding workgroup at n = 32 fetches
-// its next tile into registers during the current tile's refinement.  A_m is
-// read a second time for its refinement (A_{m+1}'s loads are issued before
-// A_m's refinement starts where registers allow); keeping the whole tile in
-// registers through the factorisation instead exceeds 256 VGPRs and spills.
+// ---- n <= 16: one 16 x 16 product holds P = 16 / S matrices, S = 4, 8 or 16 --
+//
+// The A operand stacks P matrices' rows (lane (r = lane % 16, q = lane / 16)
+// holds row r % S of matrix r / S) and the B operand their columns, so D's
+// diagonal S x S blocks are the P products and the rest is never used.  Only
+// values of k below 4 T exist: T = ceil(n / 4) matrix instructions.
+template <int N>
+struct RefinedSmall {
+  static constexpr int S = N <= 4 ? 4 : (N <= 8 ? 8 : 16);
+  static constexpr int P = 16 / S;         // matrices per product
+  static constexpr int T = (N + 3) / 4;    // steps; step t lets lane group q stand for k = T q + t
+};
+
+// A operand of matrices m .. m + P - 1 of the tile at `a` (the last `valid`
+// matrix stands in for those past the batch; their results are not stored).
+template <int N>
+__device__ __forceinline__ void refined_small_load(const float* __restrict__ a, int m, int valid,
+                                                   float (&v)[RefinedSmall<N>::T], bool vec, int lane) {
+  using Z = RefinedSmall<N>;
+  const int r = (lane & 15) % Z::S, mm = min(m + (lane & 15) / Z::S, valid - 1), k0 = Z::T * (lane >> 4);
+  const float* const row = a + mm * (N * N) + r * N + k0;
+  if (N == 16 && vec) {
+    const f32x4 c = *reinterpret_cast<const f32x4*>(row);
+#pragma unroll
+    for (int t = 0; t < Z::T; ++t) v[t] = c[t];
+  } else {
+#pragma unroll
+    for (int t = 0; t < Z::T; ++t) v[t] = (r < N && (N % 4 == 0 || k0 + t < N)) ? row[t] : 0.0f;
+  }
+}
+
+// One refinement step of the product whose first X starts at xm (LDS, matrix
+// stride MS, row stride LD).  Every read of X precedes the first write.
+template <int N, int L>
+__device__ __forceinline__ void refined_small_step(const float (&av)[RefinedSmall<N>::T], float* xm, int lane) {
+  using G = Geo<N, L>;
+  using Z = RefinedSmall<N>;
+  const int r = lane & 15, q = lane >> 4, rs = r % Z::S;
+  float* const mine = xm + (r / Z::S) * G::MS;  // matrix of this lane's row and column
+  auto at = [&](int i, int j) {  // X[i][j], zero outside the block; see x_at
+    const bool in = i < N && j < N;
+    const float v = mine[(in ? i : 0) * G::LD + (in ? j : 0)];
+    return in ? v : 0.0f;
+  };
+  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int t = 0; t < Z::T; ++t)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(av[t]), static_cast<double>(at(Z::T * q + t, rs)),
+                                               acc, 0, 0, 0);
+  // acc[v] of this lane is D[q + 4 v][r]; of the lane's own block it has the
+  // rows q + 4 w, w = 0 .. S / 4 - 1 (those below n within the first T):
+  // E = D - I there, rounded to FP32.
+  float ee[Z::T];
+#pragma unroll
+  for (int w = 0; w < Z::T; ++w) {
+    double d = acc[w];
+#pragma unroll
+    for (int p = 1; p < Z::P; ++p) d = (r / Z::S == p) ? acc[p * (Z::S / 4) + w] : d;
+    ee[w] = static_cast<float>(d - (q + 4 * w == rs ? 1.0 : 0.0));
+  }
+  // C = X E: step w lets lane group q stand for k = q + 4 w of the block.
+  f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int w = 0; w < Z::T; ++w) c = __builtin_amdgcn_mfma_f32_16x16x4f32(at(rs, q + 4 * w), ee[w], c, 0, 0, 0);
+  // c[v] is C[4 q + v][r]: row (4 q + v) % S of matrix (4 q + v) / S
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int i = 4 * q + v;
+    if (i / Z::S == r / Z::S && i % Z::S < N && rs < N) mine[(i % Z::S) * G::LD + rs] -= c[v];
+  }
+}
+
+// The step for a whole tile in LDS, A's tile at `a`: the next product's A is
+// loaded before the current one's step.  (Two or four products interleaved
+// were slower, 142 and 159 us against 131 for 300k n = 12: fewer waves fit.)
+template <int N, int L>
+__device__ __forceinline__ void refined_small_tile(const float* __restrict__ a, float* lds, int valid, bool vec,
+                                                   int lane) {
+  using G = Geo<N, L>;
+  using Z = RefinedSmall<N>;
+  float av[Z::T];
+  refined_small_load<N>(a, 0, valid, av, vec, lane);
+#pragma unroll
+  for (int m = 0; m < G::MPW; m += Z::P) {
+    float an[Z::T];
+    if (m + Z::P < G::MPW) refined_small_load<N>(a, m + Z::P, valid, an, vec, lane);
+    refined_small_step<N, L>(av, lds + m * G::MS, lane);
+#pragma unroll
+    for (int t = 0; t < Z::T; ++t) av[t] = an[t];
+  }
+}
+
+// Lanes per matrix: the plain kernel's default (results do not depend on it).
+template <int N>
+constexpr int kRfLanes = N <= 12 ? 4 : 16;
+
+// The "rule" of the kernel that refines the X it is given instead of inverting A.
+constexpr int kPivGiven = -1;
+
+// Out-of-place inverse + one refinement step of `batch` n x n matrices: A is
+// only read, X receives the refined inverse, piv (nullable) the pivot vectors
+// (kPivGiven: X is refined in place).  `vec`: bit 0, A is 16-byte aligned;
+// bit 1, X is.  One workgroup (one wave) per tile, striding when the grid is
+// capped; a striding workgroup at n = 32 fetches its next tile into registers
+// during the current tile's refinement.  A_m is read a second time for its
+// refinement (A_{m+1}'s loads are issued before A_m's refinement starts where
+// registers allow); keeping the whole tile in registers through the
+// factorisation instead exceeds 256 VGPRs and spills.
+// Against copy + inversion + a refinement pass with every matrix padded to
+// 32 x 32 (300k matrices): n = 12 0.131 ms instead of 0.71, n = 16 0.175, n = 8
+// 0.045.  Bound at n = 12 by the matrix cores' 288 cycles per matrix (35 us)
+// on top of the plain inversion's 54 us, and the chain of each step.
 template <int N, int PIV>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void lu_refined_kernel(
     const float* __restrict__ A, float* __restrict__ X, int* __restrict__ piv, int64_t batch, int64_t ntiles,
     int vec) {
-  static_assert(N >= 17 && N <= 32, "the fused refinement takes the 16-lane layout with two rows per lane");
-  using G = Geo<N, 16>;
+  constexpr int L = kRfLanes<N>;
+  using G = Geo<N, L>;
   constexpr int NN = N * N;
+  constexpr bool small = N <= 16;
   __shared__ __attribute__((aligned(16))) float lds[G::LDS_FLOATS];
   const int lane = threadIdx.x;
-  const int l = lane % 16, g = lane / 16;
+  const int l = lane % L, g = lane / L;
   const int64_t stride = gridDim.x;
-  auto full = [&](int64_t t) { return (vec & 1) != 0 && (t + 1) * G::MPW <= batch; };
-  TileRegs<N, 16> next;
+  const float* const src = PIV == kPivGiven ? X : A;  // what is staged
+  const bool avec = (vec & 1) != 0;
+  auto full = [&](int64_t t) { return (vec & (PIV == kPivGiven ? 2 : 1)) != 0 && (t + 1) * G::MPW <= batch; };
+  TileRegs<N, L> next;
   int64_t t = blockIdx.x;
   bool have = t < ntiles && full(t);
-  if (have) tile_fetch<N, 16, false>(A + t * G::MPW * NN, next, lane);
+  if (have) tile_fetch<N, L, PIV == kPivGiven>(src + t * G::MPW * NN, next, lane);
   for (; t < ntiles; t += stride) {
     const int64_t m0 = t * G::MPW;
     const int64_t left = batch - m0;
     const int valid = left < G::MPW ? static_cast<int>(left) : G::MPW;
+    const float* const a = A + m0 * NN;
+    RefinedA am;
+    if constexpr (PIV == kPivGiven && !small) refined_load_a<N>(a, am, avec, lane);
     if (have) {
-      tile_stage<N, 16>(next, lds, lane);
+      tile_stage<N, L>(next, lds, lane);
     } else {
-      tile_load_elementwise<N, 16>(A + m0 * NN, lds, valid, lane);
+      tile_load_elementwise<N, L>(src + m0 * NN, lds, valid, lane);
     }
     wave_sync();
-    int prm[G::R];
-    RefinedA am;
-    {
-      float w[G::R][N];
-      tile_front<N, 16, PIV>(w, prm, lds, lane);
-      // A_0's second read is in flight during the elimination
-      if constexpr (kRfEarly<N>) refined_load_a<N>(A + m0 * NN, am, (vec & 1) != 0, lane);
-      tile_solve<N, 16>(w, prm, lds, lane);
-    }
-    if (piv != nullptr && g < valid) {
+    if constexpr (PIV == kPivGepp) {
+      int prm[G::R];
+      tile_gepp<N, L>(prm, lds, lane, nullptr);
+      if (piv != nullptr && g < valid) {
 #pragma unroll
-      for (int h = 0; h < G::R; ++h)
-        if (l + 16 * h < N) piv[(m0 + g) * N + l + 16 * h] = prm[h];
+        for (int h = 0; h < G::R; ++h)
+          if (l + L * h < N) piv[(m0 + g) * N + l + L * h] = prm[h];
+      }
+    } else if constexpr (PIV != kPivGiven) {
+      int prm[G::R];
+      float w[G::R][N];
+      tile_front<N, L, PIV>(w, prm, lds, lane);
+      // A_0's second read is in flight during the elimination
+      if constexpr (!small && kRfEarly<N>) refined_load_a<N>(a, am, avec, lane);
+      tile_solve<N, L>(w, prm, lds, lane);
+      if (piv != nullptr && g < valid) {
+#pragma unroll
+        for (int h = 0; h < G::R; ++h)
+          if (l + L * h < N) piv[(m0 + g) * N + l + L * h] = prm[h];
+      }
     }
     // the next tile's HBM reads overlap this tile's refinement
     const int64_t tn = t + stride;
     have = tn < ntiles && full(tn);
     if constexpr (kRfNextTile<N>) {
-      if (have) tile_fetch<N, 16, false>(A + tn * G::MPW * NN, next, lane);
+      if (have) tile_fetch<N, L, PIV == kPivGiven>(src + tn * G::MPW * NN, next, lane);
     }
-    if constexpr (!kRfEarly<N>) refined_load_a<N>(A + m0 * NN, am, (vec & 1) != 0, lane);
+    if constexpr (small) {
+      refined_small_tile<N, L>(a, lds, valid, avec, lane);
+    } else {
+      // Opaque after partial pivoting: keeps the refinement's loads and
+      // lane-derived addresses from being live through it (they would spill).
+      int ln = lane;
+      if constexpr (PIV == kPivGepp) asm volatile("" : "+v"(ln));
+      if constexpr (PIV == kPivGepp || (PIV != kPivGiven && !kRfEarly<N>)) refined_load_a<N>(a, am, avec, ln);
 #pragma unroll
-    for (int m = 0; m < G::MPW; ++m) {
-      if (m < valid) {
-        if constexpr (kRfAhead<N>) {
-          RefinedA an;
-          if (m + 1 < valid) refined_load_a<N>(A + (m0 + m + 1) * NN, an, (vec & 1) != 0, lane);
-          refined_step<N>(am, lds + m * G::MS, lane);
-          am = an;
-        } else {
-          refined_step<N>(am, lds + m * G::MS, lane);
-          if (m + 1 < valid) refined_load_a<N>(A + (m0 + m + 1) * NN, am, (vec & 1) != 0, lane);
+      for (int m = 0; m < G::MPW; ++m) {
+        if (m < valid) {
+          if constexpr (kRfAhead<N>) {
+            RefinedA an;
+            if (m + 1 < valid) refined_load_a<N>(a + (m + 1) * NN, an, avec, ln);
+            refined_step<N>(am, lds + m * G::MS, ln);
+            am = an;
+          } else {
+            refined_step<N>(am, lds + m * G::MS, ln);
+            if (m + 1 < valid) refined_load_a<N>(a + (m + 1) * NN, am, avec, ln);
+          }
         }
       }
     }
-    tile_store<N, 16>(X + m0 * NN, lds, valid, (vec & 2) != 0, lane);
+    wave_sync();
+    tile_store<N, L>(X + m0 * NN, lds, valid, (vec & 2) != 0, lane);
     wave_sync();  // the tile's region is rewritten by the next tile
     if constexpr (!kRfNextTile<N>) {
-      if (have) tile_fetch<N, 16, false>(A + tn * G::MPW * NN, next, lane);
+      if (have) tile_fetch<N, L, PIV == kPivGiven>(src + tn * G::MPW * NN, next, lane);
     }
   }
 }

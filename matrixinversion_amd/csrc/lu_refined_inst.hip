@@ -1,6 +1,7 @@
 // lu_refined_inst.hip -- instantiates lu_refined_kernel<N, PIV> (inverse +
-// one refinement step in one kernel) for N in [LUB_RF_LO, LUB_RF_HI] and the
-// pivot rules none and first-max, and registers the host handles.  Compiled
+// one refinement step in one kernel, and the refinement of a given inverse)
+// for N in [LUB_RF_LO, LUB_RF_HI] and every pivot rule, and registers the
+// host handles.  Compiled
 // once per size range so the units build in parallel.
 #include "lu_refined.hpp"
 #include "lub_internal.h"
@@ -18,8 +19,12 @@ namespace {
 template <int N>
 void register_range(lub::KernelTable* t) {
   if constexpr (N <= LUB_RF_HI) {
-    t->refined[N][0] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivNone>);
-    t->refined[N][1] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivParallel>);
+    t->refine[N] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivGiven>);
+    t->refined[N][lub::kPivNone] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivNone>);
+    t->refined[N][lub::kPivParallel] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivParallel>);
+    t->refined[N][lub::kPivSerial] = t->refined[N][lub::kPivParallel];  // the same pivots
+    t->refined[N][lub::kPivTree] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivTree>);
+    t->refined[N][lub::kPivGepp] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivGepp>);
     register_range<N + 1>(t);
   }
 }

@@ -20,8 +20,8 @@ struct KernelTable {
   // n % 4 == 0: the same kernels with the row padding flipped from its default
   const void* plain_flip[kMaxN + 1][kNumPivot][kNumLayout];
   const void* ragged[kNumPivot];
-  // inverse + one refinement step (n = 17..32): [n][0] no pivoting, [n][1] first-max
-  const void* refined[kMaxN + 1][2];
+  const void* refined[kMaxN + 1][kNumPivot];  // inverse + one refinement step
+  const void* refine[kMaxN + 1];              // one refinement step of a given inverse
 };
 
 // Per-n launch choices shared by the plain and the ragged paths (set by the
@@ -60,5 +60,9 @@ extern "C" void lub_register_ragged_0(lub::KernelTable* t);
 extern "C" void lub_register_ragged_1(lub::KernelTable* t);
 extern "C" void lub_register_ragged_3(lub::KernelTable* t);
 extern "C" void lub_register_ragged_4(lub::KernelTable* t);
-extern "C" void lub_register_refined_17_24(lub::KernelTable* t);
-extern "C" void lub_register_refined_25_32(lub::KernelTable* t);
+extern "C" void lub_register_refined_1_12(lub::KernelTable* t);
+extern "C" void lub_register_refined_13_18(lub::KernelTable* t);
+extern "C" void lub_register_refined_19_23(lub::KernelTable* t);
+extern "C" void lub_register_refined_24_27(lub::KernelTable* t);
+extern "C" void lub_register_refined_28_30(lub::KernelTable* t);
+extern "C" void lub_register_refined_31_32(lub::KernelTable* t);
