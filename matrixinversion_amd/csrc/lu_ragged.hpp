@@ -89,10 +89,10 @@ __host__ __device__ constexpr int64_t ragged_grab_limit(int64_t tiles) {
   return tiles / kRaggedTilesPerGrab > 1 ? tiles / kRaggedTilesPerGrab : 1;
 }
 
-// Batches of up to kRaggedDirectMax matrices skip the plan: each matrix gets
-// a wave of its own (a 16-lane row of it), all resident at once (8 waves per
-// CU).  256 matrices: 12.6 us against 15.6 with the plan, 1,000: 13.1 / 16.7.
-constexpr int64_t kRaggedDirectMax = 2048;
+// Batches of up to kRaggedDirectMax (lub_internal.h) matrices skip the plan:
+// each matrix gets a wave of its own (a 16-lane row of it), all resident at
+// once (8 waves per CU).  256 matrices: 12.6 us against 15.6 with the plan,
+// 1,000: 13.1 / 16.7.
 
 __host__ __device__ constexpr int ragged_mpw(int n, int layout) { return (layout == 1 && n <= kRaggedQuadMaxN) ? 16 : 4; }
 
@@ -378,7 +378,8 @@ __device__ __forceinline__ void ragged_dispatch(const RaggedDesc& d, const Ragge
 // grid makes the waves persistent.
 // With `direct_ns` (the batch's own size array; soffs and spoffs are then its
 // offset arrays) there is no plan: descriptor t is matrix t alone, and
-// descriptor `batch` counts the matrices with n outside 1..32.
+// descriptor `batch` (if the grid has one: hdr not null) counts the matrices
+// with n outside 1..32.
 template <int PIV>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void lu_ragged_kernel(
     float* __restrict__ A, const int64_t* __restrict__ soffs, int* __restrict__ piv,
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
   __shared__ __attribute__((aligned(16))) float lds[kRaggedLdsFloats];
   const int lane = threadIdx.x;
   RaggedClasses cls{};
-  int total = batch + 1;
+  int total = hdr != nullptr ? batch + 1 : batch;
   if (direct_ns == nullptr) {
     cls = ragged_load_classes(hdr, lane);
     total = __builtin_amdgcn_readlane(cls.desc_first, 0);
@@ -401,7 +402,13 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
       if (d.n < 1 || d.n > 32) continue;
     } else {
       int bad = 0;
-      for (int i = lane; i < batch; i += kWave) bad += (direct_ns[i] < 1 || direct_ns[i] > 32) ? 1 : 0;
+      for (int i0 = 0; i0 < batch; i0 += 8 * kWave) {
+        int v[8];  // eight reads in flight: one after the other they would outlast the inversions
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = direct_ns[min(i0 + k * kWave + lane, batch - 1)];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) bad += (i0 + k * kWave + lane < batch && (v[k] < 1 || v[k] > 32)) ? 1 : 0;
+      }
       for (int s = kWave / 2; s > 0; s >>= 1) bad += __shfl_xor(bad, s);
       if (lane == 0) hdr[RaggedWs::META + 2] = bad;
       continue;

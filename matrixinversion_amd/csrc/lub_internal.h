@@ -42,6 +42,15 @@ constexpr int8_t initial_pad(int n) { return (n > 0 && n % 4 == 0 && n != 28) ? 
 Tuning current_tuning();
 const KernelTable& kernel_table();
 
+// Ragged batches of up to this many matrices run without a plan.
+constexpr int64_t kRaggedDirectMax = 2048;
+
+// The ragged inversion without a plan (batch <= kRaggedDirectMax, arguments
+// checked).  The three arrays may be pinned host memory.  hdr (nullable): the
+// planning header that receives the count of matrices with n outside 1..32.
+int enqueue_ragged_direct(int* hdr, float* A, const int64_t* offsets, const int* ns, int* piv,
+                          const int64_t* piv_offsets, int64_t batch, int flags, void* stream);
+
 // The plain launch behind lu_batched_inverse_async64; info (nullable, one int
 // per matrix) receives 0 or 1 + the first step with an exactly zero pivot.
 int enqueue_plain(float* A, int* piv, int* info, int n, int64_t batch, int flags, void* stream);

@@ -232,6 +232,23 @@ __global__ __launch_bounds__(kSmallPlanThreads) void ragged_plan_small(const int
 
 }  // namespace lub
 
+namespace lub {
+
+int enqueue_ragged_direct(int* hdr, float* A, const int64_t* offsets, const int* ns, int* piv,
+                          const int64_t* piv_offsets, int64_t batch, int flags, void* stream) {
+  const void* fn = kernel_table().ragged[flags & LUB_PIVOT_MASK];
+  if (fn == nullptr) return LUB_ENODEVICE;
+  if (piv == nullptr) piv_offsets = nullptr;
+  int count = static_cast<int>(batch);
+  int layout = (flags & LUB_LAYOUT_MASK) == LUB_LAYOUT_QUAD4 ? 1 : 0;
+  void* args[] = {&A, &offsets, &piv, &piv_offsets, &hdr, &ns, &count, &layout};
+  const unsigned grid = static_cast<unsigned>(hdr != nullptr ? batch + 1 : batch);
+  return hipLaunchKernel(fn, dim3(grid), dim3(64), args, 0, static_cast<hipStream_t>(stream)) == hipSuccess ? LUB_OK
+                                                                                                         : LUB_EHIP;
+}
+
+}  // namespace lub
+
 namespace {
 
 constexpr int64_t kMaxRaggedBatch = (int64_t(1) << 31) - 64;
@@ -322,17 +339,10 @@ int enqueue_ragged(char* ws, int64_t capacity, int cus, float* A, const int64_t*
   int* bhist = reinterpret_cast<int*>(ws + lub::RaggedWs::bhist_offset());
   int64_t* soffs = reinterpret_cast<int64_t*>(ws + lub::RaggedWs::slots_offset(capacity));
   int64_t* spoffs_all = soffs + capacity;
+  if (batch <= lub::kRaggedDirectMax)
+    return lub::enqueue_ragged_direct(hdr, A, offsets, ns, piv, piv_offsets, batch, flags, s);
   const int* direct_ns = nullptr;
-  int count = static_cast<int>(batch);
-  int direct_layout = (flags & LUB_LAYOUT_MASK) == LUB_LAYOUT_QUAD4 ? 1 : 0;
-  if (batch <= lub::kRaggedDirectMax) {
-    const int64_t* no_plan_offs = offsets;
-    const int64_t* no_plan_poffs = piv ? piv_offsets : nullptr;
-    direct_ns = ns;
-    void* args[] = {&A, &no_plan_offs, &piv, &no_plan_poffs, &hdr, &direct_ns, &count, &direct_layout};
-    const hipError_t e = hipLaunchKernel(fn, dim3(static_cast<unsigned>(batch + 1)), dim3(64), args, 0, s);
-    return e == hipSuccess ? LUB_OK : LUB_EHIP;
-  }
+  int count = static_cast<int>(batch), direct_layout = 0;
   if (batch <= lub::kSmallPlanMax) {
     lub::ragged_plan_small<<<1, lub::kSmallPlanThreads, 0, s>>>(ns, offsets, piv ? piv_offsets : nullptr, batch, hdr,
                                                                 rt, soffs, spoffs_all);

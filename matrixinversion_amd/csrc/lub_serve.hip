@@ -21,9 +21,11 @@
 //   progress  retires batches whose completion event has fired, then, while a
 //             launch slot is free, launches the queued requests of a pivot
 //             rule (the front run of its ring) as one ragged batch on that
-//             slot: the batch's slot entries go up in one copy per array, the
-//             slot's stream waits for the copies, runs the ragged plan and
-//             records the batch's completion event.  Batches on different
+//             slot: the slot's stream waits for the requests' copies, inverts
+//             the batch and records its completion event.  A batch that needs
+//             no plan (up to 2,048 matrices) reads its slot entries from the
+//             pinned staging ring; a larger one gets them in one copy per
+//             array first.  Batches on different
 //             slots -- of one rule or of several -- run concurrently.
 //   poll      the tickets finished since the last poll, in completion order.
 //   query     state, device result pointers and end-to-end latency (host clock,
@@ -41,6 +43,7 @@
 #include <new>
 #include <vector>
 
+#include "lub_internal.h"
 #include "lubatch.h"
 #include "lubatch_util.h"
 
@@ -95,6 +98,9 @@ struct Rule {
   int64_t* h_offs = nullptr;      // pinned staging ring
   int* h_ns = nullptr;
   int64_t* h_poffs = nullptr;
+  int64_t* m_offs = nullptr;      // the staging ring as the device addresses it
+  int* m_ns = nullptr;
+  int64_t* m_poffs = nullptr;
   int64_t head = 0, tail = 0;     // monotonic slot positions
   std::deque<uint64_t> queued;    // tickets in submission order
   std::deque<RingRun> runs;       // launched batches not yet reclaimed
@@ -156,6 +162,10 @@ int rule_init(lub_server* s, Rule& r) {
   if (hipHostMalloc(&r.h_offs, n * 8, hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&r.h_ns, n * 4, hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&r.h_poffs, n * 8, hipHostMallocDefault) != hipSuccess)
+    return LUB_EHIP;
+  if (hipHostGetDevicePointer(reinterpret_cast<void**>(&r.m_offs), r.h_offs, 0) != hipSuccess ||
+      hipHostGetDevicePointer(reinterpret_cast<void**>(&r.m_ns), r.h_ns, 0) != hipSuccess ||
+      hipHostGetDevicePointer(reinterpret_cast<void**>(&r.m_poffs), r.h_poffs, 0) != hipSuccess)
     return LUB_EHIP;
   return LUB_OK;
 }
@@ -241,19 +251,26 @@ int launch(lub_server* s, int rule, Slot& sl, int* launched) {
     end += rq->count;
     ++take;
   }
-  // the batch's slot entries in one upload per array (staged by submit)
+  // The batch's slot entries, staged by submit.  Each of a small batch's waves
+  // reads its own from host memory (20 bytes, two round trips of a few us);
+  // the three uploads would occupy the copy stream, where the requests' own
+  // data waits, for longer.
   const int64_t at = begin % s->ring;
   const size_t cnt = static_cast<size_t>(end - begin);
-  if (hipMemcpyAsync(r.d_offs + at, r.h_offs + at, cnt * 8, hipMemcpyHostToDevice, s->copy) != hipSuccess ||
-      hipMemcpyAsync(r.d_ns + at, r.h_ns + at, cnt * 4, hipMemcpyHostToDevice, s->copy) != hipSuccess ||
-      hipMemcpyAsync(r.d_poffs + at, r.h_poffs + at, cnt * 8, hipMemcpyHostToDevice, s->copy) != hipSuccess)
+  const bool direct = end - begin <= lub::kRaggedDirectMax;
+  if (!direct &&
+      (hipMemcpyAsync(r.d_offs + at, r.h_offs + at, cnt * 8, hipMemcpyHostToDevice, s->copy) != hipSuccess ||
+       hipMemcpyAsync(r.d_ns + at, r.h_ns + at, cnt * 4, hipMemcpyHostToDevice, s->copy) != hipSuccess ||
+       hipMemcpyAsync(r.d_poffs + at, r.h_poffs + at, cnt * 8, hipMemcpyHostToDevice, s->copy) != hipSuccess))
     return LUB_EHIP;
   if (hipEventRecord(sl.copied, s->copy) != hipSuccess) return LUB_EHIP;
   if (hipStreamWaitEvent(sl.stream, sl.copied, 0) != hipSuccess) return LUB_EHIP;
   float* A = reinterpret_cast<float*>(s->arena);
   int* piv = rule == LUB_PIVOT_NONE ? nullptr : reinterpret_cast<int*>(s->arena);
-  int rc = lu_batched_inverse_ragged_plan(sl.plan, A, r.d_offs + at, r.d_ns + at, piv,
-                                          piv ? r.d_poffs + at : nullptr, end - begin, flags, sl.stream);
+  int rc = direct ? lub::enqueue_ragged_direct(nullptr, A, r.m_offs + at, r.m_ns + at, piv, r.m_poffs + at,
+                                               end - begin, flags, sl.stream)
+                  : lu_batched_inverse_ragged_plan(sl.plan, A, r.d_offs + at, r.d_ns + at, piv,
+                                                   piv ? r.d_poffs + at : nullptr, end - begin, flags, sl.stream);
   if (rc != LUB_OK) return rc;  // the inversion kernel did not start: the batch can run again later
   // From here the batch is committed (its matrices are being inverted in
   // place, so it must never be launched a second time).

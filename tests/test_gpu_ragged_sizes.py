@@ -67,3 +67,36 @@ def test_every_plan_rule_matches_plain(gpu, pools, mode, flags, batch):
     assert np.array_equal(x.view(np.uint32), want.view(np.uint32))
     assert np.array_equal(p, pwant)
     assert count == bad.size
+
+
+@pytest.mark.parametrize("mode,flags", [("parallel", 0x1), ("none", 0x0)])
+def test_server_batches_around_the_plan_limit(gpu, pools, mode, flags):
+    """A server batch of up to 2,048 matrices takes its slot entries from
+    pinned host memory, a larger one from the device: same results, also when
+    the ring has wrapped."""
+    from matrixinversion_amd import serve
+
+    pool = pools[mode]
+    rng = np.random.RandomState(5 + flags)
+    with serve.Server(64 << 20, max_batch=4096, ring_slots=5000) as srv:
+        for count in (1, 2047, 2048, 2049, 300, 4096, 700):
+            ns = rng.randint(1, 33, count).astype(np.int32)
+            pick = rng.randint(0, PER_N, count)
+            src = gpu.DeviceBuffer.from_array(np.concatenate([pool[n][0][k].ravel() for n, k in zip(ns, pick)]))
+            want = np.concatenate([pool[n][1][k].ravel() for n, k in zip(ns, pick)])
+            pwant = np.concatenate([pool[n][2][k] for n, k in zip(ns, pick)])
+            print(f"[case] serve mode={mode} count={count}", flush=True)
+            t = srv.submit(src.ptr, ns, flags)
+            assert t is not None
+            for _ in range(1000000):
+                srv.progress()
+                if t in srv.poll():
+                    break
+            state, res, piv, _ = srv.query(t)
+            assert state == serve.DONE
+            got = serve.download(res, want.nbytes, np.float32)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+            if piv:
+                assert np.array_equal(serve.download(piv, pwant.size * 4, np.int32), pwant)
+            srv.release(t)
+            src.close()
