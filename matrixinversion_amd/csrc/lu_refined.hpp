@@ -8,8 +8,8 @@
 // its inverse is the FP32 LU result (parallel_pivot/luBatchedInplace.cuh:
 // 84-125, stored at :194-197).
 //
-// Per tile (one wave; 16 lanes per matrix and 4 matrices for n > 12, quads
-// and 16 matrices up to n = 12, as in the plain kernel):
+// Per tile (one wave; 16 lanes per matrix and 4 matrices, or quads and 16
+// matrices, as in the plain kernel):
 //   1. the tile arrives in registers (TileRegs) and is staged into LDS;
 //   2. tile_front + tile_solve (tile_gepp) leave X = A^-1 in the tile's LDS
 //      region; the form that refines a given X (kPivGiven) stages X instead;
@@ -281,10 +281,6 @@ __device__ __forceinline__ void refined_small_tile(const float* __restrict__ a, 
   }
 }
 
-// Lanes per matrix: the plain kernel's default (results do not depend on it).
-template <int N>
-constexpr int kRfLanes = N <= 12 ? 4 : 16;
-
 // The "rule" of the kernel that refines the X it is given instead of inverting A.
 constexpr int kPivGiven = -1;
 
@@ -301,11 +297,10 @@ constexpr int kPivGiven = -1;
 // 32 x 32 (300k matrices): n = 12 0.131 ms instead of 0.71, n = 16 0.175, n = 8
 // 0.045.  Bound at n = 12 by the matrix cores' 288 cycles per matrix (35 us)
 // on top of the plain inversion's 54 us, and the chain of each step.
-template <int N, int PIV>
+template <int N, int L, int PIV>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void lu_refined_kernel(
     const float* __restrict__ A, float* __restrict__ X, int* __restrict__ piv, int64_t batch, int64_t ntiles,
     int vec) {
-  constexpr int L = kRfLanes<N>;
   using G = Geo<N, L>;
   constexpr int NN = N * N;
   constexpr bool small = N <= 16;

@@ -16,15 +16,28 @@
 
 namespace {
 
+template <int N, int L, int PIV>
+const void* handle() {
+  return reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, L, PIV>);
+}
+
+template <int N, int L>
+void register_layout(lub::KernelTable* t, int layout) {
+  t->refine[N][layout] = handle<N, L, lub::kPivGiven>();
+  auto& slot = t->refined[N];
+  slot[lub::kPivNone][layout] = handle<N, L, lub::kPivNone>();
+  slot[lub::kPivParallel][layout] = handle<N, L, lub::kPivParallel>();
+  slot[lub::kPivSerial][layout] = slot[lub::kPivParallel][layout];  // the same pivots
+  slot[lub::kPivTree][layout] = handle<N, L, lub::kPivTree>();
+  if constexpr (L == 16 || N <= lub::kGeppQuadMaxN) slot[lub::kPivGepp][layout] = handle<N, L, lub::kPivGepp>();
+}
+
+// The layouts that refined_layout() of the entry points picks.
 template <int N>
 void register_range(lub::KernelTable* t) {
   if constexpr (N <= LUB_RF_HI) {
-    t->refine[N] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivGiven>);
-    t->refined[N][lub::kPivNone] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivNone>);
-    t->refined[N][lub::kPivParallel] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivParallel>);
-    t->refined[N][lub::kPivSerial] = t->refined[N][lub::kPivParallel];  // the same pivots
-    t->refined[N][lub::kPivTree] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivTree>);
-    t->refined[N][lub::kPivGepp] = reinterpret_cast<const void*>(&lub::lu_refined_kernel<N, lub::kPivGepp>);
+    if constexpr (N > lub::kGeppQuadMaxN) register_layout<N, 16>(t, 0);
+    if constexpr (N <= lub::kRefinedQuadMaxN) register_layout<N, 4>(t, 1);
     register_range<N + 1>(t);
   }
 }

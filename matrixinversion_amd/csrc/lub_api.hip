@@ -39,7 +39,8 @@ const lub::KernelTable& table() {
     lub_register_ragged_1(&g_table);
     lub_register_ragged_3(&g_table);
     lub_register_ragged_4(&g_table);
-    lub_register_refined_1_12(&g_table);
+    lub_register_refined_1_8(&g_table);
+    lub_register_refined_9_12(&g_table);
     lub_register_refined_13_18(&g_table);
     lub_register_refined_19_23(&g_table);
     lub_register_refined_24_27(&g_table);
@@ -131,7 +132,7 @@ int default_layout(int n) {
   return (g_tuning.layout[n] == 1 && n <= lub::kLayoutMaxN[1]) ? 1 : 0;
 }
 
-int choose_layout(int n, int flags) {
+int choose_layout(int n, int flags, int64_t batch) {
   switch (flags & LUB_LAYOUT_MASK) {
     case LUB_LAYOUT_ROW16: return 0;
     case LUB_LAYOUT_QUAD4: return 1;
@@ -140,6 +141,7 @@ int choose_layout(int n, int flags) {
   static int forced = env_int("LUB_LANES");
   if (forced == 4 && n <= lub::kLayoutMaxN[1]) return 1;
   if (forced == 16) return 0;
+  if (lub::rows_beat_quads(n, (flags & LUB_PIVOT_MASK) == LUB_PIVOT_GEPP, batch)) return 0;
   return default_layout(n);
 }
 
@@ -168,7 +170,7 @@ const KernelTable& kernel_table() { return table(); }
 int enqueue_plain(float* A, int* piv, int* info, int n, int64_t batch, int flags, void* stream) {
   int rc = validate(A, piv, n, batch, flags);
   if (rc != LUB_OK || batch == 0) return rc;
-  const int layout = choose_layout(n, flags);
+  const int layout = choose_layout(n, flags, batch);
   bool flip = false;
   if (n % 4 == 0) {
     std::lock_guard<std::mutex> lock(g_tuning_mutex);

@@ -20,8 +20,9 @@ struct KernelTable {
   // n % 4 == 0: the same kernels with the row padding flipped from its default
   const void* plain_flip[kMaxN + 1][kNumPivot][kNumLayout];
   const void* ragged[kNumPivot];
-  const void* refined[kMaxN + 1][kNumPivot];  // inverse + one refinement step
-  const void* refine[kMaxN + 1];              // one refinement step of a given inverse
+  // [layout]: inverse + one refinement step, and the step for a given inverse
+  const void* refined[kMaxN + 1][kNumPivot][kNumLayout];
+  const void* refine[kMaxN + 1][kNumLayout];
 };
 
 // Per-n launch choices shared by the plain and the ragged paths (set by the
@@ -40,6 +41,20 @@ constexpr int8_t geo_pad(int n) { return (n > 0 && n % 8 == 0) ? 1 : 0; }
 // 4 % and 9 % of the kernel time, at n = 28 it costs 7 %).
 constexpr int8_t initial_pad(int n) { return (n > 0 && n % 4 == 0 && n != 28) ? 1 : 0; }
 Tuning current_tuning();
+
+// Where the table's quads give way to 16-lane rows under LUB_LAYOUT_AUTO.
+// Partial pivoting holds rows, and a quad's lane would hold three of them
+// from n = 9 (four from n = 13): the pivot row's selection and its masked LDS
+// stores then cost several times the update (100k matrices, quads / rows: n =
+// 8 14 / 21 us, n = 9 85 / 25, n = 12 229 / 38).  The other rules' chains are
+// longer in quads too, which shows only while the chip is not full: 4,096
+// matrices of n = 12 4.9 / 3.9 us, 16,384 6.8 / 6.9, 100k 23 / 25.
+constexpr int kGeppQuadMaxN = 8;
+constexpr int64_t kSmallBatchQuads = 8192;
+constexpr int kRefinedQuadMaxN = 12;  // the refined kernels' quads
+constexpr bool rows_beat_quads(int n, bool gepp, int64_t batch) {
+  return n > kGeppQuadMaxN && (gepp || batch <= kSmallBatchQuads);
+}
 const KernelTable& kernel_table();
 
 // Ragged batches of up to this many matrices run without a plan.
@@ -69,7 +84,8 @@ extern "C" void lub_register_ragged_0(lub::KernelTable* t);
 extern "C" void lub_register_ragged_1(lub::KernelTable* t);
 extern "C" void lub_register_ragged_3(lub::KernelTable* t);
 extern "C" void lub_register_ragged_4(lub::KernelTable* t);
-extern "C" void lub_register_refined_1_12(lub::KernelTable* t);
+extern "C" void lub_register_refined_1_8(lub::KernelTable* t);
+extern "C" void lub_register_refined_9_12(lub::KernelTable* t);
 extern "C" void lub_register_refined_13_18(lub::KernelTable* t);
 extern "C" void lub_register_refined_19_23(lub::KernelTable* t);
 extern "C" void lub_register_refined_24_27(lub::KernelTable* t);

@@ -330,6 +330,7 @@ int enqueue_ragged(char* ws, int64_t capacity, int cus, float* A, const int64_t*
   lub::RaggedTuning rt;
   for (int n = 0; n <= 32; ++n) {
     int layout = tuning.layout[n];
+    if (pv == LUB_PIVOT_GEPP && lub::rows_beat_quads(n, true, batch)) layout = 0;
     if ((flags & LUB_LAYOUT_MASK) == LUB_LAYOUT_ROW16) layout = 0;
     if ((flags & LUB_LAYOUT_MASK) == LUB_LAYOUT_QUAD4) layout = 1;
     rt.layout[n] = static_cast<int8_t>(layout);

@@ -27,10 +27,18 @@ int check_args(const float* A, float* X, int n, int64_t batch) {
   return -1;  // proceed
 }
 
+// Lane layout: quads up to n = 12 unless rows are faster.  A tile of quads
+// takes its 16 matrices' steps one after the other, so the small-batch line
+// lies higher than the plain kernel's.
+int refined_layout(int n, bool gepp, int64_t batch) {
+  if (n > lub::kRefinedQuadMaxN) return 0;
+  return lub::rows_beat_quads(n, gepp, batch / 2) ? 0 : 1;
+}
+
 // One workgroup per tile (several tiles per workgroup measured slower).
-int enqueue(const void* fn, const float* A, float* X, int* piv, int n, int64_t batch, void* stream) {
+int enqueue(const void* fn, int layout, const float* A, float* X, int* piv, int64_t batch, void* stream) {
   if (fn == nullptr) return LUB_ENODEVICE;
-  const int per_tile = n <= 12 ? 16 : 4;  // matrices (kRfLanes)
+  const int per_tile = 64 / lub::kLayoutLanes[layout];  // matrices
   int64_t ntiles = (batch + per_tile - 1) / per_tile;
   const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ntiles, int64_t(1) << 22));
   int vec = ((reinterpret_cast<uintptr_t>(A) & 15u) == 0 ? 1 : 0) | ((reinterpret_cast<uintptr_t>(X) & 15u) == 0 ? 2 : 0);
@@ -46,7 +54,8 @@ extern "C" {
 int lu_batched_refine(const float* A, float* X, int n, int64_t batch, void* stream) {
   const int rc = check_args(A, X, n, batch);
   if (rc >= 0) return rc;
-  return enqueue(lub::kernel_table().refine[n], A, X, nullptr, n, batch, stream);
+  const int layout = refined_layout(n, false, batch);
+  return enqueue(lub::kernel_table().refine[n][layout], layout, A, X, nullptr, batch, stream);
 }
 
 int lu_batched_inverse_refined(const float* A, float* X, int* piv, int n, int64_t batch, int flags, void* stream) {
@@ -59,7 +68,8 @@ int lu_batched_inverse_refined(const float* A, float* X, int* piv, int n, int64_
     return LUB_EFLAGS;
   const bool any_piv = n >= 17 && (rule == LUB_PIVOT_NONE || rule == LUB_PIVOT_PARALLEL || rule == LUB_PIVOT_SERIAL);
   if (!any_piv && (reinterpret_cast<uintptr_t>(piv) & 3u) != 0) return LUB_EALIGN;
-  return enqueue(lub::kernel_table().refined[n][rule], A, X, piv, n, batch, stream);
+  const int lanes = refined_layout(n, rule == LUB_PIVOT_GEPP, batch);
+  return enqueue(lub::kernel_table().refined[n][rule][lanes], lanes, A, X, piv, batch, stream);
 }
 
 }  // extern "C"
