@@ -51,41 +51,43 @@ constexpr bool kRfAhead = N <= 28 || N == 32;
 template <int N>
 constexpr bool kRfNextTile = N == 32;
 
+// Values of k per lane group in the FP64 product of n = 17..32: step t lets
+// group q stand for k = T q + t, so n / 4 steps suffice.
+template <int N>
+constexpr int kRfSteps = (N + 3) / 4;
+
 // A_m in the FP64 product's operand layout: lane (r = lane % 16,
-// q = lane / 16) holds A_m[16 I + r][8 q + t], I = 0, 1, t = 0..7, and zero
+// q = lane / 16) holds A_m[16 I + r][T q + t], I = 0, 1, t = 0..T-1, and zero
 // outside the n x n block.
+template <int N>
 struct RefinedA {
-  float v[2][8];
+  float v[2][kRfSteps<N>];
 };
 
 // Loads A_m (matrix at `a`) with ordinary loads: the tile's first read used
 // them too, so this second read is normally served from the caches.  `vec`:
-// the batch is 16-byte aligned (n % 4 == 0 then reads 16-byte chunks).
+// the batch is 16-byte aligned (n = 32 then reads 16-byte chunks; other n
+// read the T consecutive floats of a row at their own alignment).
 template <int N>
-__device__ __forceinline__ void refined_load_a(const float* __restrict__ a, RefinedA& r, bool vec, int lane) {
+__device__ __forceinline__ void refined_load_a(const float* __restrict__ a, RefinedA<N>& r, bool vec, int lane) {
+  constexpr int T = kRfSteps<N>;
   const int r16 = lane & 15, q = lane >> 4;
 #pragma unroll
   for (int I = 0; I < 2; ++I) {
     const int i = 16 * I + r16;
-    if constexpr (N % 4 == 0) {
+    const float* const row = a + i * N + T * q;
+    if (N == 32 && vec) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int j = 8 * q + 4 * h;  // n % 4 == 0: a chunk lies wholly inside or outside the block
-        f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (N == 32 || (i < N && j < N)) {
-          if (vec) {
-            c = *reinterpret_cast<const f32x4*>(a + i * N + j);
-          } else {
-            c = f32x4{a[i * N + j], a[i * N + j + 1], a[i * N + j + 2], a[i * N + j + 3]};
-          }
-        }
-        r.v[I][4 * h] = c.x; r.v[I][4 * h + 1] = c.y; r.v[I][4 * h + 2] = c.z; r.v[I][4 * h + 3] = c.w;
+        const f32x4 c = *reinterpret_cast<const f32x4*>(row + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[I][4 * h + e] = c[e];
       }
     } else {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int j = 8 * q + t;
-        r.v[I][t] = (i < N && j < N) ? a[i * N + j] : 0.0f;
+      for (int t = 0; t < T; ++t) {
+        const bool in = (N == 32 || I == 0 || i < N) && (N % 4 == 0 || T * q + t < N);
+        r.v[I][t] = in ? row[t] : 0.0f;
       }
     }
   }
@@ -110,12 +112,12 @@ __device__ __forceinline__ float x_at(const float* xm, int i, int j) {
 // X_m in the tile's LDS region (row stride Geo::LD), where the refined X_m
 // replaces it (every read of X_m precedes the first write).
 template <int N>
-__device__ __forceinline__ void refined_step(const RefinedA& am, float* xm, int lane) {
+__device__ __forceinline__ void refined_step(const RefinedA<N>& am, float* xm, int lane) {
   constexpr int LD = Geo<N, 16>::LD;
   const int r16 = lane & 15, q = lane >> 4;
   // D = A_m X_m on the FP64 matrix cores, four 16 x 16 blocks (I, J).  In
   // v_mfma_f64_16x16x4f64 operand lane l holds A[l % 16][kk] and X[kk][l % 16]
-  // with kk = l / 16; step t lets lane group q stand for k = 8 q + t, so A_m's
+  // with kk = l / 16; step t lets lane group q stand for k = T q + t, so A_m's
   // registers are used as loaded.  Accumulator element v of lane l is
   // D[16 I + l / 16 + 4 v][16 J + l % 16].
   f64x4 acc[2][2];
@@ -124,8 +126,8 @@ __device__ __forceinline__ void refined_step(const RefinedA& am, float* xm, int 
 #pragma unroll
     for (int J = 0; J < 2; ++J) acc[I][J] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const int k = 8 * q + t;
+  for (int t = 0; t < kRfSteps<N>; ++t) {
+    const int k = kRfSteps<N> * q + t;
     double xv[2];
 #pragma unroll
     for (int J = 0; J < 2; ++J) {
@@ -169,6 +171,7 @@ __device__ __forceinline__ void refined_step(const RefinedA& am, float* xm, int 
   for (int I = 0; I < 2; ++I)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
+      if (16 * I + 4 * v >= N) continue;  // rows of E past n
       const int k = 16 * I + q + 4 * v;
       float xa[2];
 #pragma unroll
@@ -320,7 +323,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
     const int64_t left = batch - m0;
     const int valid = left < G::MPW ? static_cast<int>(left) : G::MPW;
     const float* const a = A + m0 * NN;
-    RefinedA am;
+    RefinedA<N> am;
     if constexpr (PIV == kPivGiven && !small) refined_load_a<N>(a, am, avec, lane);
     if (have) {
       tile_stage<N, L>(next, lds, lane);
@@ -367,7 +370,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
       for (int m = 0; m < G::MPW; ++m) {
         if (m < valid) {
           if constexpr (kRfAhead<N>) {
-            RefinedA an;
+            RefinedA<N> an;
             if (m + 1 < valid) refined_load_a<N>(a + (m + 1) * NN, an, avec, ln);
             refined_step<N>(am, lds + m * G::MS, ln);
             am = an;
