@@ -79,14 +79,15 @@ constexpr int kRaggedMaxPer = 64;  // matrices per descriptor: one slot per lane
 
 // The tuned grab amortises a descriptor's start-up where the chip is full;
 // in a small batch it would only chain tiles in one wave while compute units
-// idle.  So a descriptor takes no more than 1 / kRaggedTilesPerGrab of the
-// batch's tiles.  Mixed n = 4..32, us for grab 1 / 2 / 4 / 8 / the table (8,
-// 4 and 16): 3,000 matrices 20 / 28 / 44 / 77 / 131; 32,768 50 / 50 / 58 / 89
-// / 145; 100,000 (19k tiles) 113 / 109 / 115 / 123 / 175.  From 64k tiles
-// (about 350,000 such matrices) the table's 8 stands.
-constexpr int kRaggedTilesPerGrab = 8192;
-__host__ __device__ constexpr int64_t ragged_grab_limit(int64_t tiles) {
-  return tiles / kRaggedTilesPerGrab > 1 ? tiles / kRaggedTilesPerGrab : 1;
+// idle.  So a descriptor takes no more than 1 / 4096 of the batch's tiles, or
+// 1 / 2048 where a tile is short (n <= 16).  n = 4..32 mixed, us for grab 1 /
+// 2 / 4 / 8 / the table (8, 4 and 16): 3,000 matrices 20 / 28 / 44 / 77 / 131;
+// 32,768 50 / 50 / 58 / 89 / 145; 100,000 (19k tiles) 113 / 109 / 115 / 123 /
+// 175.  From 33k tiles the table's 8 stands: 160,000 of n = 1..23 (24k tiles)
+// 138 with 3 and 7, 133 with 8.
+__host__ __device__ constexpr int ragged_grab_limit(int n, int tiles) {
+  const int limit = tiles / (n <= 16 ? 2048 : 4096);
+  return limit > 1 ? limit : 1;
 }
 
 // Batches of up to kRaggedDirectMax (lub_internal.h) matrices skip the plan:
@@ -256,24 +257,29 @@ __device__ __forceinline__ void ragged_tile(float* __restrict__ A, int* __restri
                                             int count, float* lds, int lane) {
   using G = Geo<N, L, 1>;
   static_assert(G::LDS_FLOATS <= kRaggedLdsFloats, "tile exceeds the ragged kernel's LDS array");
-  const int l = lane % L;
-  const int g = lane / L;
   RaggedRegs<N, L> x;
   ragged_load<N, L>(A, sl, 0, min(G::MPW, count), x, lane);
   for (int base = 0;;) {
     const int valid = min(G::MPW, count - base);
-    ragged_stage<N, L>(x, valid, lds, lane);
+    // Partial pivoting needs the registers: opaque before and after it, the
+    // lane's addresses are formed where they are used instead of staying live
+    // through the elimination (155 spilled registers; 500k n = 28..32 2.24 ms).
+    int ln = lane;
+    if constexpr (PIV == kPivGepp) asm volatile("" : "+v"(ln));
+    ragged_stage<N, L>(x, valid, lds, ln);
     wave_sync();
     LaneInts<N, L> prm;
     if constexpr (PIV == kPivGepp) {
-      tile_gepp<N, L, 1>(prm, lds, lane, nullptr);
+      tile_gepp<N, L, 1>(prm, lds, ln, nullptr);
+      asm volatile("" : "+v"(ln));
     } else {
       ColBlock<N, L> w;
       tile_front<N, L, PIV, 1>(w, prm, lds, lane);
       tile_solve<N, L, 1>(w, prm, lds, lane);
     }
     auto finish = [&](int b0, int nv) {
-      ragged_scatter_store<N, L>(A, sl, b0, nv, lds, lane);
+      const int l = ln % L, g = ln / L;
+      ragged_scatter_store<N, L>(A, sl, b0, nv, lds, ln);
       if (piv != nullptr) {
         const int64_t po = slot_lane(sl.po_lo, sl.po_hi, b0 + (g < nv ? g : 0));
         if (g < nv) {
@@ -288,7 +294,7 @@ __device__ __forceinline__ void ragged_tile(float* __restrict__ A, int* __restri
     // the staged ones are dead during the factorisation.
     const int nb = base + G::MPW;
     if (nb < count) {
-      ragged_load<N, L>(A, sl, nb, min(G::MPW, count - nb), x, lane);
+      ragged_load<N, L>(A, sl, nb, min(G::MPW, count - nb), x, ln);
       finish(base, valid);
       base = nb;
     } else {
