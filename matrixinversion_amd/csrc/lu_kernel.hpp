@@ -56,6 +56,8 @@ constexpr int kWave = 64;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+// A float4 at any float offset: gfx950 executes dword-aligned dwordx4.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 enum Pivot : int { kPivNone = 0, kPivParallel = 1, kPivSerial = 2, kPivTree = 3, kPivGepp = 4 };
 
@@ -208,11 +210,11 @@ __device__ __forceinline__ void lds_row_write(float* p, const float (&w)[N]) {
 
 // ------------------------------------------------------------- tile I/O
 
-// HBM -> LDS.  Full tiles of a 16-byte aligned batch move as dwordx4 chunks
-// (chunk c = floats 4c..4c+3 of the tile), fetched into registers (TileRegs)
-// and staged into LDS.  The last, partial tile and unaligned batches move
-// element-wise, and matrices past the end of the batch are filled with the
-// identity so every lane computes on finite data.
+// HBM -> LDS.  Tiles move as dwordx4 chunks (chunk c = floats 4c..4c+3 of the
+// tile), fetched into registers (TileRegs) and staged into LDS: full tiles of
+// a 16-byte aligned batch by tile_fetch, unaligned ones and the last, partial
+// tile by tile_fetch_part; matrices past the end of the batch are filled with
+// the identity so every lane computes on finite data.
 template <int N, int L>
 struct TileRegs {
   static constexpr int CH = Geo<N, L>::MPW * N * N / 4;  // dwordx4 chunks per tile
@@ -282,13 +284,44 @@ __device__ __forceinline__ void tile_stage(const TileRegs<N, L>& r, float* lds, 
   }
 }
 
+// The leading `lim` floats of a tile at any 4-byte alignment (gfx950 executes
+// dword-aligned dwordx4), zeros after them.  A loop over single floats, each
+// load waited for, took 4-5 us of a small launch: 100 matrices of n = 12 (16
+// per tile) 8.6 us against 4.7 for 512, one of n = 32 15.2 against 9.2 for four.
+template <int N, int L, bool NT = true>
+__device__ __forceinline__ void tile_fetch_part(const float* __restrict__ src, TileRegs<N, L>& r, int lim, int lane) {
+  using T = TileRegs<N, L>;
+  // opaque: nothing of this seldom-run path is computed ahead of the tile loop
+  // into registers that would stay live (and spill) through the elimination
+  asm volatile("" : "+v"(lane));
+#pragma unroll
+  for (int it = 0; it < T::IT; ++it) {
+    const int f = 4 * (lane + kWave * it);
+    f32x4u v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (f + 4 <= lim) {
+      if constexpr (NT) v = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(src + f));
+      else v = *reinterpret_cast<const f32x4u*>(src + f);
+    } else {
+      if (f < lim) v[0] = src[f];
+      if (f + 1 < lim) v[1] = src[f + 1];
+      if (f + 2 < lim) v[2] = src[f + 2];
+    }
+    r.v[it] = f32x4{v[0], v[1], v[2], v[3]};
+  }
+}
+
+// A partial tile: the registers of tile_fetch_part staged, and the diagonal
+// of the matrices past the batch set to one.
 template <int N, int L, int V = 0>
-__device__ __forceinline__ void tile_load_elementwise(const float* __restrict__ src, float* lds, int valid, int lane) {
+__device__ __forceinline__ void tile_identity(float* lds, int valid, int lane) {
   using G = Geo<N, L, V>;
-  constexpr int NN = N * N;
-  for (int f = lane; f < G::MPW * NN; f += kWave) {
-    const int m = f / NN, e = f - m * NN, i = e / N, j = e - i * N;
-    lds[m * G::MS + i * G::LD + j] = (m < valid) ? src[f] : (i == j ? 1.0f : 0.0f);
+  asm volatile("" : "+v"(lane));  // see tile_fetch_part
+  const int l = lane % L, g = lane / L;
+  wave_sync();  // after the staging of their zeros
+  if (g >= valid) {
+#pragma unroll
+    for (int h = 0; h < G::R; ++h)
+      if (l + L * h < N) lds[g * G::MS + (l + L * h) * (G::LD + 1)] = 1.0f;
   }
 }
 
@@ -297,7 +330,6 @@ template <int N, int L, int V = 0>
 __device__ __forceinline__ void tile_store(float* __restrict__ dst, const float* lds, int valid, bool vec, int lane) {
   using G = Geo<N, L, V>;
   using T = TileRegs<N, L>;
-  constexpr int NN = N * N;
   if (vec && valid == G::MPW) {
     const int base = chunk_lds_base<N, L, V>(lane);
 #pragma unroll
@@ -309,9 +341,21 @@ __device__ __forceinline__ void tile_store(float* __restrict__ dst, const float*
       }
     }
   } else {
-    for (int f = lane; f < valid * NN; f += kWave) {
-      const int m = f / NN, e = f - m * NN, i = e / N, j = e - i * N;
-      dst[f] = lds[m * G::MS + i * G::LD + j];
+    asm volatile("" : "+v"(lane));  // see tile_fetch_part
+    const int lim = valid * (N * N), base = chunk_lds_base<N, L, V>(lane);
+#pragma unroll
+    for (int it = 0; it < T::IT; ++it) {
+      const int c = lane + kWave * it, f = 4 * c;
+      if (T::CH % kWave == 0 || c < T::CH) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(lds + chunk_lds_offset<N, L, V>(base, lane, it));
+        if (f + 4 <= lim) {
+          __builtin_nontemporal_store(f32x4u{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4u*>(dst + f));
+        } else {
+          if (f < lim) dst[f] = v[0];
+          if (f + 1 < lim) dst[f + 1] = v[1];
+          if (f + 2 < lim) dst[f + 2] = v[2];
+        }
+      }
     }
   }
 }
@@ -881,8 +925,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kWavesPer
     const int64_t m0 = t * G::MPW;
     const int64_t left = batch - m0;
     const int valid = left < G::MPW ? (int)left : G::MPW;
-    if (have) tile_stage<N, L, V>(next, lds, lane);
-    else tile_load_elementwise<N, L, V>(A + m0 * (N * N), lds, valid, lane);
+    if (!have) tile_fetch_part<N, L>(A + m0 * (N * N), next, valid * (N * N), lane);
+    tile_stage<N, L, V>(next, lds, lane);
+    if (valid < G::MPW) tile_identity<N, L, V>(lds, valid, lane);
     wave_sync();
     int prm[G::R];
     if constexpr (PIV == kPivGepp) {

@@ -104,9 +104,7 @@ constexpr int cmax() { return A_ > B_ ? A_ : B_; }
 
 constexpr int kRaggedLdsFloats = cmax<Geo<32, 16, 1>::LDS_FLOATS, Geo<kRaggedQuadMaxN, 4, 1>::LDS_FLOATS>();
 
-// Float4 of a ragged batch: matrices start at any float offset, so global
-// accesses are only 4-byte aligned (gfx950 executes dword-aligned dwordx4).
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+// Matrices start at any float offset, so global accesses are f32x4u.
 
 // Slot offsets of one descriptor, one slot per lane (lanes 0..15; lanes past
 // the descriptor's count repeat slot 0): matrix offset and pivot offset.

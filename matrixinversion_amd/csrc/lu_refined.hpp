@@ -325,11 +325,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
     const float* const a = A + m0 * NN;
     RefinedA<N> am;
     if constexpr (PIV == kPivGiven && !small) refined_load_a<N>(a, am, avec, lane);
-    if (have) {
-      tile_stage<N, L>(next, lds, lane);
-    } else {
-      tile_load_elementwise<N, L>(src + m0 * NN, lds, valid, lane);
-    }
+    if (!have) tile_fetch_part<N, L, PIV == kPivGiven>(src + m0 * NN, next, valid * NN, lane);
+    tile_stage<N, L>(next, lds, lane);
+    if (valid < G::MPW) tile_identity<N, L>(lds, valid, lane);
     wave_sync();
     if constexpr (PIV == kPivGepp) {
       int prm[G::R];
