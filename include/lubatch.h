@@ -99,9 +99,9 @@ int lu_batched_inverse_async64(float* A, int* piv, int n, int64_t batch, int fla
  * A (row-major, contiguous, inverted in place); its pivot vector goes to
  * piv + piv_offsets[i] (piv may be NULL).  All five arrays are device
  * memory.  The batch is planned and inverted on the device by one
- * persistent kernel (size classes largest first, per-class lane layout and
- * matrices per work item from the tuning table); results equal a plain launch
- * of each matrix's n.  Matrices with n outside 1..32 are skipped and counted
+ * kernel (size classes largest first, per-class lane layout and matrices per
+ * work item from the tuning table; batches of up to 2048 matrices need no
+ * plan); results equal a plain launch of each matrix's n.  Matrices with n outside 1..32 are skipped and counted
  * (lu_ragged_invalid_count).  Replaces, for mixed sizes, one reference build
  * and launch per MATRIXSIZE (parallel_pivot/run.py:198-234). */
 typedef struct lub_ragged_plan lub_ragged_plan;
@@ -146,7 +146,9 @@ int lu_ragged_invalid_count(const lub_ragged_plan* plan, int* out);
  * (0 = 16-lane rows, 1 = quads; quads apply to n <= 16 in the plain kernel,
  * n <= 12 in the ragged one) and grab[n] (ragged: wave tiles per work item,
  * >= 1, used up to 64 matrices per item and less in batches too small to
- * fill the GPU that way).  Arrays of 33 entries indexed by n
+ * fill the GPU that way).  Where quads were measured slower, rows are used
+ * whatever the table holds: n >= 9 with LUB_PIVOT_GEPP, and n >= 9 in plain
+ * batches of up to 8192 matrices.  Arrays of 33 entries indexed by n
  * (entry 0 unused). */
 int lu_tuning_set(const signed char* layout, const signed char* grab);
 int lu_tuning_get(signed char* layout, signed char* grab);
