@@ -261,7 +261,8 @@ __device__ __forceinline__ void ragged_tile(float* __restrict__ A, int* __restri
     const int valid = min(G::MPW, count - base);
     // Partial pivoting needs the registers: opaque before and after it, the
     // lane's addresses are formed where they are used instead of staying live
-    // through the elimination (155 spilled registers; 500k n = 28..32 2.24 ms).
+    // through the elimination (500k n = 28..32: 1.99 ms with 8 spilled
+    // registers, 2.24 with 155).
     int ln = lane;
     if constexpr (PIV == kPivGepp) asm volatile("" : "+v"(ln));
     ragged_stage<N, L>(x, valid, lds, ln);
