@@ -110,18 +110,20 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_scan(int* __restrict__ ws
   }
 }
 
-// The class table from the class totals: classes 32, 31, ..., 1 in order;
-// a descriptor holds MPW(n) * grab(n) matrices, at most kRaggedMaxPer (one
-// slot per lane), so grab is clamped to 16 with 16-lane rows and 4 with
-// quads, and to ragged_grab_limit of the batch's tiles.  Every scatter block derives it (32 values); block 0 publishes it
-// in the header for the inversion kernel.
-__device__ void ragged_class_table(int* __restrict__ ws, int64_t batch, const RaggedTuning& tune, bool publish,
-                                   int* first_slot) {
+// The class table from the class totals counts[1..32] (written before the
+// caller's last barrier, or by an earlier kernel): classes 32, 31, ..., 1 in
+// order; a descriptor holds MPW(n) * grab(n) matrices, at most kRaggedMaxPer
+// (one slot per lane), so grab is clamped to 16 with 16-lane rows and 4 with
+// quads, and to ragged_grab_limit of the batch's tiles.  Every scatter block
+// derives it (32 values); block 0 publishes it in the header for the
+// inversion kernel.
+__device__ __forceinline__ void ragged_class_table(const int* counts, int* ws, int64_t batch, const RaggedTuning& tune,
+                                                   bool publish, int* first_slot) {
   const int t = threadIdx.x;
   if (t < kWave) {  // the first wave: lane t < 32 has class 32 - t, so prefixes run from n = 32 down
     const int c = 32 - t;
     const bool row = t < 32;
-    const int cnt = row ? ws[RaggedWs::COUNTS + c] : 0;
+    const int cnt = row ? counts[c] : 0;
     const int layout = (row && tune.layout[row ? c : 0] == 1 && c <= kRaggedQuadMaxN) ? 1 : 0;
     const int mpw = ragged_mpw(c, layout);
     int tiles = (cnt + mpw - 1) / mpw;
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_scatter(const int* __rest
                                                                int64_t* __restrict__ spoffs) {
   __shared__ int first_slot[33];
   __shared__ int cur[33];
-  ragged_class_table(ws, batch, tune, blockIdx.x == 0, first_slot);
+  ragged_class_table(ws + RaggedWs::COUNTS, ws, batch, tune, blockIdx.x == 0, first_slot);
   const int c = threadIdx.x;
   if (c >= 1 && c <= 32) cur[c] = first_slot[c] + bhist[c * nblocks + blockIdx.x];
   __syncthreads();
@@ -210,8 +212,8 @@ __global__ __launch_bounds__(kSmallPlanThreads) void ragged_plan_small(const int
     atomicAdd(&hist[(n >= 1 && n <= 32) ? n : 0], 1);
   }
   __syncthreads();
-  if (t >= 1 && t <= 32) ws[RaggedWs::COUNTS + t] = hist[t];  // read back below by the same thread
-  ragged_class_table(ws, batch, tune, true, first_slot);
+  if (t >= 1 && t <= 32) ws[RaggedWs::COUNTS + t] = hist[t];  // for the inversion kernel
+  ragged_class_table(hist, ws, batch, tune, true, first_slot);
   if (t >= 1 && t <= 32) cur[t] = first_slot[t];
   __syncthreads();
   for (int64_t i = t; i < batch; i += kSmallPlanThreads) {
