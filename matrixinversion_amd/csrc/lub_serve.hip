@@ -25,8 +25,9 @@
 //             the batch and records its completion event.  A batch that needs
 //             no plan (up to 2,048 matrices) reads its slot entries from the
 //             pinned staging ring; a larger one gets them in one copy per
-//             array first.  Batches on different
-//             slots -- of one rule or of several -- run concurrently.
+//             array first.  Batches on different slots -- of one rule or of
+//             several -- run concurrently; only behind a short batch of its
+//             own rule does a request wait, and gather with others (kGather).
 //   poll      the tickets finished since the last poll, in completion order.
 //   query     state, device result pointers and end-to-end latency (host clock,
 //             submit to the progress call that saw the batch complete).
@@ -55,6 +56,19 @@ constexpr int kRules = 5;                 // LUB_PIVOT_NONE .. LUB_PIVOT_GEPP
 constexpr int kSlots = 3;                 // batches in flight at once (+ the copy stream = 4 streams)
 constexpr int64_t kAlign = 256;           // request blocks start on 256-byte boundaries
 
+// While a batch of at most kGather matrices (8,192 row tiles, one filling of
+// the chip: about 0.1 ms) of a rule runs, further requests of the rule gather
+// until it is done or kGather matrices wait.  A launch (event, wait, launch,
+// event) costs the host some 20 us, a batch of a few requests ends in about
+// as much, so without this a burst becomes one launch per request and is bound
+// by them.  First-max, us per burst / batches: 64 requests of 1,000 of n =
+// 24..32 1,268 / 8 with, 2,570 / 64 without; 64 of 64 of n = 4..32 1,388 / 18
+// and 2,512 / 64; 32 of 2,000 726 / 5 and 1,318 / 32.  Limits of 2,048 and
+// 16,384 leave larger requests behind (64 of 2,000: 1,981 and 1,629 against
+// 1,370).  A Poisson stream of 16,000 requests/s pays for it in its median
+// (0.056-0.060 -> 0.064-0.072 ms), one of 64,000 gains (0.16 -> 0.135).
+constexpr int64_t kGather = 32768;
+
 int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
 enum State : int { kQueued = 0, kRunning = 1, kDone = 2 };
@@ -81,6 +95,7 @@ struct Slot {
   hipEvent_t done = nullptr;     // the batch is inverted
   bool busy = false;
   int rule = -1;
+  int64_t count = 0;             // matrices of the batch
   int64_t ring_end = 0;          // monotonic ring position after the batch
   std::vector<uint64_t> tickets;
 };
@@ -233,6 +248,15 @@ int retire(lub_server* s, int* completed) {
   return LUB_OK;
 }
 
+// Whether `rule`'s queued requests wait for more (see kGather).
+bool gathering(lub_server* s, int rule) {
+  const Rule& r = s->rules[rule];
+  if (r.head - find(s, r.queued.front())->slot >= std::min(kGather, s->max_batch)) return false;
+  for (const Slot& sl : s->slots)
+    if (sl.busy && sl.rule == rule && sl.count <= kGather) return true;
+  return false;
+}
+
 // Launch the front run of `rule`'s queue on `sl`.  Tickets leave the queue
 // only once every enqueue has succeeded; on an error they stay queued (and
 // the slot stays free), so a later progress call retries them.
@@ -254,7 +278,8 @@ int launch(lub_server* s, int rule, Slot& sl, int* launched) {
   // The batch's slot entries, staged by submit.  Each of a small batch's waves
   // reads its own from host memory (20 bytes, two round trips of a few us);
   // the three uploads would occupy the copy stream, where the requests' own
-  // data waits, for longer.
+  // data waits, for longer (8 requests of 64: 229 us a burst; uploaded 295,
+  // with or without a plan; at no size up to 2,000 per request slower).
   const int64_t at = begin % s->ring;
   const size_t cnt = static_cast<size_t>(end - begin);
   const bool direct = end - begin <= lub::kRaggedDirectMax;
@@ -286,6 +311,7 @@ int launch(lub_server* s, int rule, Slot& sl, int* launched) {
   }
   sl.busy = true;
   sl.rule = rule;
+  sl.count = end - begin;
   sl.ring_end = end;
   r.runs.push_back(RingRun{end, false});
   ++r.inflight;
@@ -395,13 +421,13 @@ int lu_server_progress(lub_server* s, int* launched, int* completed) {
   if (completed) *completed = 0;
   int rc = retire(s, completed);
   if (rc != LUB_OK) return rc;
-  // Free slots go to the rules with queued work, the rule with the fewest
+  // Free slots go to the rules with work to launch, the rule with the fewest
   // batches running first (ties: lower rule number).
   for (Slot& sl : s->slots) {
     if (sl.busy) continue;
     int pick = -1;
     for (int rule = 0; rule < kRules; ++rule) {
-      if (s->rules[rule].queued.empty()) continue;
+      if (s->rules[rule].queued.empty() || gathering(s, rule)) continue;
       if (pick < 0 || s->rules[rule].inflight < s->rules[pick].inflight) pick = rule;
     }
     if (pick < 0) break;
