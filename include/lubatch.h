@@ -147,9 +147,9 @@ int lu_ragged_invalid_count(const lub_ragged_plan* plan, int* out);
  * n <= 12 in the ragged one) and grab[n] (ragged: wave tiles per work item,
  * >= 1, used up to 64 matrices per item and less in batches too small to
  * fill the GPU that way).  Where quads were measured slower, rows are used
- * whatever the table holds: n >= 9 with LUB_PIVOT_GEPP, and n >= 9 in plain
- * batches of up to 8192 matrices.  Arrays of 33 entries indexed by n
- * (entry 0 unused). */
+ * whatever the table holds: n >= 9 with LUB_PIVOT_GEPP, and n = 9..12 in
+ * batches of up to 8192 matrices (16384 in lu_batched_inverse_refined).
+ * Arrays of 33 entries indexed by n (entry 0 unused). */
 int lu_tuning_set(const signed char* layout, const signed char* grab);
 int lu_tuning_get(signed char* layout, signed char* grab);
 
@@ -188,8 +188,9 @@ int lu_perm_to_ipiv(int* piv, int n, int64_t batch, void* stream);
 int lu_batched_refine(const float* A, float* X, int n, int64_t batch, void* stream);
 
 /* Out-of-place inverse plus one refinement step: X <- A^-1 (the plain path
- * with `flags`, pivots to piv as in lu_batched_inverse), then
- * lu_batched_refine(A, X).  A is left unchanged (A != X). */
+ * with `flags`, pivots to piv as in lu_batched_inverse, in the layout that
+ * the flags or the table name), then lu_batched_refine(A, X).  A is left
+ * unchanged (A != X). */
 int lu_batched_inverse_refined(const float* A, float* X, int* piv, int n, int64_t batch, int flags, void* stream);
 
 /* ---- serving ------------------------------------------------------------

@@ -1,8 +1,8 @@
-// lu_refined_inst.hip -- instantiates lu_refined_kernel<N, PIV> (inverse +
+// lu_refined_inst.hip -- instantiates lu_refined_kernel<N, L, PIV> (inverse +
 // one refinement step in one kernel, and the refinement of a given inverse)
-// for N in [LUB_RF_LO, LUB_RF_HI] and every pivot rule, and registers the
-// host handles.  Compiled
-// once per size range so the units build in parallel.
+// for N in [LUB_RF_LO, LUB_RF_HI], every pivot rule and the layouts of the
+// plain kernel (16-lane rows, quads up to n = 16), and registers the host
+// handles.  Compiled once per size range so the units build in parallel.
 #include "lu_refined.hpp"
 #include "lub_internal.h"
 
@@ -23,21 +23,22 @@ const void* handle() {
 
 template <int N, int L>
 void register_layout(lub::KernelTable* t, int layout) {
-  t->refine[N][layout] = handle<N, L, lub::kPivGiven>();
   auto& slot = t->refined[N];
   slot[lub::kPivNone][layout] = handle<N, L, lub::kPivNone>();
   slot[lub::kPivParallel][layout] = handle<N, L, lub::kPivParallel>();
   slot[lub::kPivSerial][layout] = slot[lub::kPivParallel][layout];  // the same pivots
   slot[lub::kPivTree][layout] = handle<N, L, lub::kPivTree>();
-  if constexpr (L == 16 || N <= lub::kGeppQuadMaxN) slot[lub::kPivGepp][layout] = handle<N, L, lub::kPivGepp>();
+  slot[lub::kPivGepp][layout] = handle<N, L, lub::kPivGepp>();
 }
 
-// The layouts that refined_layout() of the entry points picks.
 template <int N>
 void register_range(lub::KernelTable* t) {
   if constexpr (N <= LUB_RF_HI) {
-    if constexpr (N > lub::kGeppQuadMaxN) register_layout<N, 16>(t, 0);
-    if constexpr (N <= lub::kRefinedQuadMaxN) register_layout<N, 4>(t, 1);
+    register_layout<N, 16>(t, 0);
+    if constexpr (N <= lub::kLayoutMaxN[1]) register_layout<N, 4>(t, 1);
+    // the two that lu_batched_refine picks from
+    if constexpr (N > lub::kGeppQuadMaxN) t->refine[N][0] = handle<N, 16, lub::kPivGiven>();
+    if constexpr (N <= lub::kRefineQuadMaxN) t->refine[N][1] = handle<N, 4, lub::kPivGiven>();
     register_range<N + 1>(t);
   }
 }

@@ -132,19 +132,6 @@ int default_layout(int n) {
   return (g_tuning.layout[n] == 1 && n <= lub::kLayoutMaxN[1]) ? 1 : 0;
 }
 
-int choose_layout(int n, int flags, int64_t batch) {
-  switch (flags & LUB_LAYOUT_MASK) {
-    case LUB_LAYOUT_ROW16: return 0;
-    case LUB_LAYOUT_QUAD4: return 1;
-    default: break;
-  }
-  static int forced = env_int("LUB_LANES");
-  if (forced == 4 && n <= lub::kLayoutMaxN[1]) return 1;
-  if (forced == 16) return 0;
-  if (lub::rows_beat_quads(n, (flags & LUB_PIVOT_MASK) == LUB_PIVOT_GEPP, batch)) return 0;
-  return default_layout(n);
-}
-
 int validate(const float* A, const int* piv, int n, int64_t batch, int flags) {
   if (n < 1 || n > LUB_MAX_N) return LUB_EINVAL_N;
   if (batch < 0) return LUB_EINVAL_BATCH;
@@ -165,6 +152,19 @@ Tuning current_tuning() {
   return g_tuning;
 }
 const KernelTable& kernel_table() { return table(); }
+
+int choose_layout(int n, int flags, int64_t batch, int64_t small_batch) {
+  switch (flags & LUB_LAYOUT_MASK) {
+    case LUB_LAYOUT_ROW16: return 0;
+    case LUB_LAYOUT_QUAD4: return 1;
+    default: break;
+  }
+  static int forced = env_int("LUB_LANES");
+  if (forced == 4 && n <= kLayoutMaxN[1]) return 1;
+  if (forced == 16) return 0;
+  if (rows_beat_quads(n, (flags & LUB_PIVOT_MASK) == LUB_PIVOT_GEPP, batch, small_batch)) return 0;
+  return default_layout(n);
+}
 
 // The plain launch; info (nullable) receives LAPACK-style per-matrix info.
 int enqueue_plain(float* A, int* piv, int* info, int n, int64_t batch, int flags, void* stream) {

@@ -46,15 +46,26 @@ Tuning current_tuning();
 // Partial pivoting holds rows, and a quad's lane would hold three of them
 // from n = 9 (four from n = 13): the pivot row's selection and its masked LDS
 // stores then cost several times the update (100k matrices, quads / rows: n =
-// 8 14 / 21 us, n = 9 85 / 25, n = 12 229 / 38).  The other rules' chains are
-// longer in quads too, which shows only while the chip is not full: 4,096
-// matrices of n = 12 4.9 / 3.9 us, 16,384 6.8 / 6.9, 100k 23 / 25.
+// 8 14 / 21 us, n = 9 85 / 25, n = 12 229 / 38, n = 16 514 / 59).  The other
+// rules' chains are longer in quads too, which shows only while the chip is
+// not full: 4,096 matrices of n = 12 4.9 / 3.9 us, 16,384 6.8 / 6.9, 100k
+// 23 / 25.  The initial table has quads up to n = 12; one that has them above
+// is taken at its word.
 constexpr int kGeppQuadMaxN = 8;
+constexpr int kSmallBatchMaxN = 12;
 constexpr int64_t kSmallBatchQuads = 8192;
-constexpr int kRefinedQuadMaxN = 12;  // the refined kernels' quads
-constexpr bool rows_beat_quads(int n, bool gepp, int64_t batch) {
-  return n > kGeppQuadMaxN && (gepp || batch <= kSmallBatchQuads);
+// The refined kernels take a quad tile's 16 matrices' steps one after the
+// other, so their line lies higher (n = 12, 16,384 matrices: 13.3 / 10.3 us;
+// 100k: 47.5 / 48.2).
+constexpr int64_t kSmallBatchRefinedQuads = 16384;
+constexpr bool rows_beat_quads(int n, bool gepp, int64_t batch, int64_t small_batch = kSmallBatchQuads) {
+  return n > kGeppQuadMaxN && (gepp || (n <= kSmallBatchMaxN && batch <= small_batch));
 }
+// Layout of a call: the one that `flags` or LUB_LANES force, else rows where
+// they beat quads, else the table's.
+int choose_layout(int n, int flags, int64_t batch, int64_t small_batch = kSmallBatchQuads);
+
+constexpr int kRefineQuadMaxN = 12;  // quads of the refinement of a given inverse
 const KernelTable& kernel_table();
 
 // Ragged batches of up to this many matrices run without a plan.

@@ -27,14 +27,6 @@ int check_args(const float* A, float* X, int n, int64_t batch) {
   return -1;  // proceed
 }
 
-// Lane layout: quads up to n = 12 unless rows are faster.  A tile of quads
-// takes its 16 matrices' steps one after the other, so the small-batch line
-// lies higher than the plain kernel's.
-int refined_layout(int n, bool gepp, int64_t batch) {
-  if (n > lub::kRefinedQuadMaxN) return 0;
-  return lub::rows_beat_quads(n, gepp, batch / 2) ? 0 : 1;
-}
-
 // One workgroup per tile (several tiles per workgroup measured slower).
 int enqueue(const void* fn, int layout, const float* A, float* X, int* piv, int64_t batch, void* stream) {
   if (fn == nullptr) return LUB_ENODEVICE;
@@ -54,7 +46,8 @@ extern "C" {
 int lu_batched_refine(const float* A, float* X, int n, int64_t batch, void* stream) {
   const int rc = check_args(A, X, n, batch);
   if (rc >= 0) return rc;
-  const int layout = refined_layout(n, false, batch);
+  const bool quads = n <= lub::kRefineQuadMaxN && !lub::rows_beat_quads(n, false, batch, lub::kSmallBatchRefinedQuads);
+  const int layout = quads ? 1 : 0;
   return enqueue(lub::kernel_table().refine[n][layout], layout, A, X, nullptr, batch, stream);
 }
 
@@ -68,8 +61,8 @@ int lu_batched_inverse_refined(const float* A, float* X, int* piv, int n, int64_
     return LUB_EFLAGS;
   const bool any_piv = n >= 17 && (rule == LUB_PIVOT_NONE || rule == LUB_PIVOT_PARALLEL || rule == LUB_PIVOT_SERIAL);
   if (!any_piv && (reinterpret_cast<uintptr_t>(piv) & 3u) != 0) return LUB_EALIGN;
-  const int lanes = refined_layout(n, rule == LUB_PIVOT_GEPP, batch);
-  return enqueue(lub::kernel_table().refined[n][rule][lanes], lanes, A, X, piv, batch, stream);
+  const int chosen = lub::choose_layout(n, flags, batch, lub::kSmallBatchRefinedQuads);
+  return enqueue(lub::kernel_table().refined[n][rule][chosen], chosen, A, X, piv, batch, stream);
 }
 
 }  // extern "C"

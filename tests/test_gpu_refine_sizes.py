@@ -67,3 +67,68 @@ def test_rough_inverse_is_corrected(gpu, n):
     scale = np.abs(ref).max(axis=(1, 2), keepdims=True)
     # the correction's n-term FP32 sums: n ulps of 1e-3 of the scale, and one rounding
     assert np.all(np.abs(got - ref) <= 2.0 ** -24 * np.abs(ref) + (n + 2) * 2.0 ** -24 * 4e-3 * scale)
+
+
+@pytest.mark.parametrize("rule", sorted(RULES))
+@pytest.mark.parametrize("n", range(1, 17))
+def test_forced_layouts_agree(gpu, n, rule):
+    """16-lane rows and quads, partial tiles and unaligned A and X: the same
+    bits, within the FP64 step of the plain inverse."""
+    from matrixinversion_amd._native import check, lib
+
+    for batch, a_off, x_off in ((64, 0, 0), (37, 4, 0), (19, 0, 4), (1, 8, 12)):
+        a = oracle.dominant_matrices(900 + n, batch, n)
+        x0, p0 = gpu.invert(a, RULES[rule])
+        guard = np.full(8, np.float32(-7.25))
+        A, X, P = gpu.DeviceBuffer(a.nbytes + 16), gpu.DeviceBuffer(a.nbytes + 48), gpu.DeviceBuffer(batch * n * 4)
+        got = []
+        try:
+            A.upload(a, offset=a_off)
+            for layout in (0x10, 0x20):
+                print(f"[case] refined n={n} rule={rule} layout={layout:#x} batch={batch} at {a_off},{x_off}", flush=True)
+                X.upload(guard, offset=x_off + a.nbytes)
+                check(lib().lu_batched_inverse_refined(A.ptr + a_off, X.ptr + x_off, P.ptr, n, batch,
+                                                       RULES[rule] | layout, None))
+                gpu.synchronize()
+                got.append(X.download(a.shape, np.float32, offset=x_off))
+                assert np.array_equal(P.download((batch, n), np.int32), p0)
+                assert np.array_equal(X.download((8,), np.float32, offset=x_off + a.nbytes), guard)
+        finally:
+            for b in (A, X, P):
+                b.close()
+        assert _within_step(a, x0, got[0])
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [9, 10, 11, 12])
+def test_quads_above_the_small_batch_line(gpu, n):
+    """From 16,385 matrices n = 9..12 take quads, in the refined inverse and in
+    the refinement of a given X: the bits of a small batch (rows), also in a
+    partial last tile and unaligned."""
+    from matrixinversion_amd._native import check, lib
+
+    block = oracle.dominant_matrices(950 + n, 512, n)
+    for batch, off in ((16385, 0), (16389, 4), (16400, 0)):
+        a = np.tile(block, (batch // 512 + 1, 1, 1))[:batch].copy()
+        x0, _ = gpu.invert(block, 0x1)
+        A, X = gpu.DeviceBuffer(a.nbytes + 4), gpu.DeviceBuffer(a.nbytes + 4)
+        try:
+            A.upload(a, offset=off)
+            for given in (False, True):
+                results = []
+                for count in (512, batch):
+                    print(f"[case] refined quads n={n} batch={count} offset={off} given={given}", flush=True)
+                    if given:
+                        X.upload(np.tile(x0, (batch // 512 + 1, 1, 1))[:batch].copy(), offset=off)
+                        check(lib().lu_batched_refine(A.ptr + off, X.ptr + off, n, count, None))
+                    else:
+                        check(lib().lu_batched_inverse_refined(A.ptr + off, X.ptr + off, None, n, count, 0x1, None))
+                    gpu.synchronize()
+                    results.append(X.download((count, n, n), np.float32, offset=off))
+                rows, quads = results
+                assert _within_step(block, x0, rows)
+                want = np.tile(rows, (batch // 512 + 1, 1, 1))[:batch]
+                assert np.array_equal(quads.view(np.uint32), want.view(np.uint32))
+        finally:
+            A.close()
+            X.close()
