@@ -148,7 +148,8 @@ int lu_ragged_invalid_count(const lub_ragged_plan* plan, int* out);
  * >= 1, used up to 64 matrices per item and less in batches too small to
  * fill the GPU that way).  Where quads were measured slower, rows are used
  * whatever the table holds: n >= 9 with LUB_PIVOT_GEPP, and n = 9..12 in
- * batches of up to 8192 matrices (16384 in lu_batched_inverse_refined).
+ * batches of up to 8192 matrices (16384 in lu_batched_inverse_refined), and
+ * in ragged batches that need no plan (a wave holds one matrix there).
  * Arrays of 33 entries indexed by n (entry 0 unused). */
 int lu_tuning_set(const signed char* layout, const signed char* grab);
 int lu_tuning_get(signed char* layout, signed char* grab);

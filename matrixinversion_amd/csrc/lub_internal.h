@@ -74,7 +74,8 @@ constexpr int64_t kRaggedDirectMax = 2048;
 // The ragged inversion without a plan (batch <= kRaggedDirectMax, arguments
 // checked).  The three arrays may be pinned host memory.  hdr (nullable): the
 // planning header that receives the count of matrices with n outside 1..32.
-int enqueue_ragged_direct(int* hdr, float* A, const int64_t* offsets, const int* ns, int* piv,
+// cus: the device's compute units (for ragged_persistent_grid).
+int enqueue_ragged_direct(int* hdr, int cus, float* A, const int64_t* offsets, const int* ns, int* piv,
                           const int64_t* piv_offsets, int64_t batch, int flags, void* stream);
 
 // The plain launch behind lu_batched_inverse_async64; info (nullable, one int

@@ -230,7 +230,17 @@ __global__ __launch_bounds__(kSmallPlanThreads) void ragged_plan_small(const int
 
 namespace lub {
 
-int enqueue_ragged_direct(int* hdr, float* A, const int64_t* offsets, const int* ns, int* piv,
+// LUB_RAGGED_WAVES_PER_CU=<k>: a grid of k persistent waves per compute unit;
+// 0 where it is not set.
+int64_t ragged_persistent_grid(int cus) {
+  static const int per_cu = [] {
+    const char* e = std::getenv("LUB_RAGGED_WAVES_PER_CU");
+    return e != nullptr ? std::atoi(e) : 0;
+  }();
+  return per_cu > 0 && cus > 0 ? int64_t(cus) * per_cu : 0;
+}
+
+int enqueue_ragged_direct(int* hdr, int cus, float* A, const int64_t* offsets, const int* ns, int* piv,
                           const int64_t* piv_offsets, int64_t batch, int flags, void* stream) {
   const void* fn = kernel_table().ragged[flags & LUB_PIVOT_MASK];
   if (fn == nullptr) return LUB_ENODEVICE;
@@ -238,7 +248,8 @@ int enqueue_ragged_direct(int* hdr, float* A, const int64_t* offsets, const int*
   int count = static_cast<int>(batch);
   int layout = (flags & LUB_LAYOUT_MASK) == LUB_LAYOUT_QUAD4 ? 1 : 0;
   void* args[] = {&A, &offsets, &piv, &piv_offsets, &hdr, &ns, &count, &layout};
-  const unsigned grid = static_cast<unsigned>(hdr != nullptr ? batch + 1 : batch);
+  const int64_t persistent = ragged_persistent_grid(cus), items = hdr != nullptr ? batch + 1 : batch;
+  const unsigned grid = static_cast<unsigned>(persistent > 0 ? std::min(persistent, items) : items);
   return hipLaunchKernel(fn, dim3(grid), dim3(64), args, 0, static_cast<hipStream_t>(stream)) == hipSuccess ? LUB_OK
                                                                                                          : LUB_EHIP;
 }
@@ -281,14 +292,9 @@ int ragged_per(const lub::RaggedTuning& rt, int n) {
 
 // Grid of the inversion kernel: by default at least the descriptor count
 // (ceil(batch / smallest matrices-per-descriptor) + 32 bounds it), so each
-// workgroup does one descriptor; LUB_RAGGED_WAVES_PER_CU=<k> launches k
-// persistent waves per compute unit instead.
+// workgroup does one descriptor; or ragged_persistent_grid.
 int64_t ragged_grid(int cus, const lub::RaggedTuning& rt, int64_t batch) {
-  static const int per_cu = [] {
-    const char* e = std::getenv("LUB_RAGGED_WAVES_PER_CU");
-    return e != nullptr ? std::atoi(e) : 0;
-  }();
-  if (per_cu > 0 && cus > 0) return int64_t(cus) * per_cu;
+  if (const int64_t persistent = lub::ragged_persistent_grid(cus); persistent > 0) return persistent;
   int min_per = lub::kRaggedMaxPer, min_mpw = lub::kRaggedMaxPer;
   for (int n = 1; n <= 32; ++n) {
     min_per = std::min(min_per, ragged_per(rt, n));
@@ -341,7 +347,7 @@ int enqueue_ragged(char* ws, int64_t capacity, int cus, float* A, const int64_t*
   int64_t* soffs = reinterpret_cast<int64_t*>(ws + lub::RaggedWs::slots_offset(capacity));
   int64_t* spoffs_all = soffs + capacity;
   if (batch <= lub::kRaggedDirectMax)
-    return lub::enqueue_ragged_direct(hdr, A, offsets, ns, piv, piv_offsets, batch, flags, s);
+    return lub::enqueue_ragged_direct(hdr, cus, A, offsets, ns, piv, piv_offsets, batch, flags, s);
   const int* direct_ns = nullptr;
   int count = static_cast<int>(batch), direct_layout = 0;
   if (batch <= lub::kSmallPlanMax) {

@@ -126,6 +126,7 @@ struct Rule {
 
 struct lub_server {
   int device = 0;
+  int cus = 0;                    // compute units of `device`
   char* arena = nullptr;
   int64_t arena_bytes = 0;
   int64_t head = 0, tail = 0;     // monotonic arena positions
@@ -292,7 +293,7 @@ int launch(lub_server* s, int rule, Slot& sl, int* launched) {
   if (hipStreamWaitEvent(sl.stream, sl.copied, 0) != hipSuccess) return LUB_EHIP;
   float* A = reinterpret_cast<float*>(s->arena);
   int* piv = rule == LUB_PIVOT_NONE ? nullptr : reinterpret_cast<int*>(s->arena);
-  int rc = direct ? lub::enqueue_ragged_direct(nullptr, A, r.m_offs + at, r.m_ns + at, piv, r.m_poffs + at,
+  int rc = direct ? lub::enqueue_ragged_direct(nullptr, s->cus, A, r.m_offs + at, r.m_ns + at, piv, r.m_poffs + at,
                                                end - begin, flags, sl.stream)
                   : lu_batched_inverse_ragged_plan(sl.plan, A, r.d_offs + at, r.d_ns + at, piv,
                                                    piv ? r.d_poffs + at : nullptr, end - begin, flags, sl.stream);
@@ -334,7 +335,9 @@ int lu_server_create(lub_server** out, int64_t budget_bytes, int64_t max_batch, 
   s->max_batch = max_batch;
   s->ring = ring_slots;
   int rc = LUB_OK;
-  if (hipGetDevice(&s->device) != hipSuccess || hipMalloc(&s->arena, s->arena_bytes) != hipSuccess ||
+  if (hipGetDevice(&s->device) != hipSuccess ||
+      hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess ||
+      hipMalloc(&s->arena, s->arena_bytes) != hipSuccess ||
       hipStreamCreateWithFlags(&s->copy, hipStreamNonBlocking) != hipSuccess)
     rc = LUB_EHIP;
   for (int i = 0; rc == LUB_OK && i < kSlots; ++i) rc = slot_init(s, s->slots[i]);

@@ -4,8 +4,16 @@ is run): forced layouts and the tuning table are honoured by the plain and the
 refined inverse, on both sides of each line where rows replace the table's
 quads."""
 import ctypes
+import os
+import subprocess
+import sys
+from types import SimpleNamespace
 
+import numpy as np
 import pytest
+
+import oracle
+from tests.conftest import ROOT
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +100,46 @@ def test_table_is_honoured(gpu, entry):
         assert _per_tile(gpu, entry, 14, 1, 100) == QUADS
     finally:
         gpu.tuning_set(layout, grab)
+
+
+def ragged_direct(gpu):
+    """(grid, inverses) of 1,500 mixed matrices, a batch that needs no plan."""
+    ns = np.random.RandomState(3).randint(1, 33, 1500).astype(np.int32)
+    flat = np.concatenate([oracle.dominant_matrices(80, 1, int(n))[0].ravel() for n in ns])
+    offs = np.concatenate([[0], np.cumsum(ns.astype(np.int64) ** 2)[:-1]])
+    A, O, NS = (gpu.DeviceBuffer.from_array(v) for v in (flat, offs, ns))
+    with gpu.RaggedPlan(ns.size) as plan:
+        print("[case] ragged without a plan, 1500 matrices", flush=True)
+        grid = _grid(gpu, lambda s: gpu.lu_batched_inverse_ragged(A, O, NS, ns.size, 0x1, plan=plan,
+                                                                  stream=SimpleNamespace(handle=s)))
+        gpu.lu_batched_inverse_ragged(A, O, NS, ns.size, 0x1, plan=plan)
+        gpu.synchronize()
+        x = A.download(flat.shape, np.float32)
+    for b in (A, O, NS):
+        b.close()
+    return grid, x
+
+
+CHILD = """
+import sys
+import numpy as np
+import matrixinversion_amd as mia
+from tests.test_gpu_layout_choice import ragged_direct
+grid, x = ragged_direct(mia)
+np.savez(sys.argv[1], grid=grid, x=x)
+"""
+
+
+def test_persistent_waves_without_a_plan(gpu, tmp_path):
+    """LUB_RAGGED_WAVES_PER_CU bounds the grid of a batch without a plan too;
+    the variable is read once, so a child process sets it."""
+    path = str(tmp_path / "direct.npz")
+    env = dict(os.environ, LUB_RAGGED_WAVES_PER_CU="1", PYTHONPATH=ROOT)
+    r = subprocess.run([sys.executable, "-u", "-c", CHILD, path], env=env, cwd=ROOT, timeout=100, capture_output=True,
+                       text=True)
+    print(r.stdout[-1000:], r.stderr[-1000:], flush=True)
+    assert r.returncode == 0
+    got = np.load(path)
+    grid, x = ragged_direct(gpu)
+    assert grid == 1501 and int(got["grid"]) == gpu.device_info(0).cu_count
+    assert np.array_equal(got["x"].view(np.uint32), x.view(np.uint32))
