@@ -1,7 +1,6 @@
 """The automatic lane layout (rows instead of quads for partial pivoting from
 n = 9 and for small batches of n = 9..12) gives the same bits as either forced
-layout, on both sides of each line, in the plain, LAPACK, ragged and refined
-entry points."""
+layout, on both sides of each line, in the plain and refined inverse."""
 import numpy as np
 import pytest
 

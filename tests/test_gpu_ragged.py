@@ -212,22 +212,28 @@ def test_ragged_large_batch_planning(gpu):
         assert _same_bits(x[gidx], flat[gidx]), f"n={n}: a skipped matrix was written"
 
 
-def test_ragged_without_pivots_and_single_class(gpu):
+@pytest.mark.parametrize("count", [70, 2500, 17000])
+def test_ragged_without_pivots_and_single_class(gpu, count):
+    """Without a plan, with the one-workgroup plan and with the three-step one."""
     rng = np.random.RandomState(4)
     for n in (1, 4, 13, 32):
         mats = _mixed("parallel", [n] * 70, seed=900 + n)
+        mats = (mats * (count // 70 + 1))[:count]
         flat, offs, ns, poffs = _pack_scattered(mats, rng)
-        print(f"[case] ragged single class n={n} no pivots", flush=True)
+        print(f"[case] ragged single class n={n} count={count} no pivots", flush=True)
         x, _ = _run_ragged(gpu, flat, offs, ns, poffs, 0x1, with_piv=False)
         xp = gpu.invert(np.stack(mats), 0x1, return_pivots=False)
         xr = np.stack([x[o:o + n * n].reshape(n, n) for o in offs])
         assert _same_bits(xr, xp)
 
 
-def test_ragged_grab_table_does_not_change_results(gpu):
+@pytest.mark.parametrize("count", [400, 4000, 60000])
+def test_ragged_grab_table_does_not_change_results(gpu, count):
+    """Tables apply from 2,049 matrices on (a batch without a plan ignores
+    them); 60,000 allow work items of two to seven tiles."""
     rng = np.random.RandomState(5)
     ns = rng.randint(1, 33, size=400)
-    mats = _mixed("parallel", ns, seed=321)
+    mats = _mixed("parallel", ns, seed=321) * (count // 400)
     flat, offs, ns32, poffs = _pack_scattered(mats, rng)
     print("[case] ragged default tuning", flush=True)
     x0, p0 = _run_ragged(gpu, flat, offs, ns32, poffs, 0x1)
@@ -246,21 +252,52 @@ def test_ragged_grab_table_does_not_change_results(gpu):
     x3, p3 = _run_ragged(gpu, flat, offs, ns32, poffs, 0x10)
     assert _same_bits(x1, x3) and (p1 == p3).all(), "grab changed row-layout results"
     assert (p2 == p0).all(), "layout choice changed pivots"
-    for i, n in enumerate(ns32):
+    for i, n in enumerate(ns32[:400]):
         e = acc.rel_err64(mats[i][None], x2[offs[i]:offs[i] + n * n].reshape(1, n, n))
         assert e[0] <= acc.contract_bound(mats[i][None], acc.rel_err64(
             mats[i][None], oracle.lu_inverse_f32(mats[i][None], oracle.PIV_FIRSTMAX)[0]))[0]
 
 
-def test_ragged_graph_replays_match_eager(gpu):
+def test_large_work_items_match_plain(gpu):
+    """Work items of up to 16 row tiles, which ragged_grab_limit allows from
+    65,536 tiles: 264,192 matrices of n = 13, 17 and 20 under several grab
+    columns, every matrix against its plain launch bit for bit."""
+    sizes, distinct, repeats = (13, 17, 20), 64, 1376
+    blocks = {n: oracle.uniform_matrices(60 + n, distinct, n) for n in sizes}
+    plain = {n: gpu.invert(blocks[n], 0x1 | 0x10) for n in sizes}
+
+    def packed(parts):  # [n][k] -> n = 13, 17, 20 of k = 0, then of k = 1, ..
+        return np.tile(np.concatenate([parts[n][k].ravel() for k in range(distinct) for n in sizes]), repeats)
+
+    ns = np.tile(np.array(sizes, np.int32), distinct * repeats)
+    offs = np.concatenate([[0], np.cumsum(ns.astype(np.int64) ** 2)[:-1]])
+    poffs = np.concatenate([[0], np.cumsum(ns.astype(np.int64))[:-1]])
+    flat, want = packed(blocks), packed({n: plain[n][0] for n in sizes})
+    pwant = packed({n: plain[n][1] for n in sizes})
+    layout, grab = gpu.tuning_get()
+    try:
+        for grabs in ((8, 8, 8), (16, 16, 16), (5, 16, 11)):
+            g = grab.copy()
+            g[list(sizes)] = grabs
+            gpu.tuning_set(layout, g)
+            print(f"[case] ragged large work items grab={grabs}", flush=True)
+            x, p = _run_ragged(gpu, flat, offs, ns, poffs, 0x1)
+            assert _same_bits(x, want) and np.array_equal(p, pwant)
+    finally:
+        gpu.tuning_set(layout, grab)
+
+
+@pytest.mark.parametrize("count", [500, 5000, 20000])
+def test_ragged_graph_replays_match_eager(gpu, count):
     """Capture (restore input; ragged inverse) on a plan once, replay it three
     times with eager work and synchronisations in between; every replay must
-    reproduce the eager result bit for bit."""
+    reproduce the eager result bit for bit.  One launch without a plan, two
+    with the one-workgroup plan, four above 16,384 matrices."""
     rng = np.random.RandomState(6)
     ns = rng.randint(1, 33, size=500)
-    mats = _mixed("parallel", ns, seed=4242)
+    mats = _mixed("parallel", ns, seed=4242) * (count // 500)
     flat, offs, ns32, poffs = _pack_scattered(mats, rng)
-    print("[case] ragged eager reference", flush=True)
+    print(f"[case] ragged eager reference count={count}", flush=True)
     x_ref, p_ref = _run_ragged(gpu, flat, offs, ns32, poffs, 0x1)
 
     src = gpu.DeviceBuffer.from_array(flat)
