@@ -119,9 +119,22 @@ def tune_pad(n: int, layout: int, batch: int, stream: Stream, reps: int = 20) ->
     return best, times
 
 
-def tune_grab(n: int, layout: int, batch: int, stream: Stream, reps: int = 20) -> tuple[int, dict]:
-    """Ragged path: wave tiles per work item for one n under `layout`."""
+def grab_candidates(n: int, layout: int, batch: int) -> list[int]:
+    """Wave tiles per work item that a ragged batch of `batch` n x n matrices
+    can tell apart: a work item holds up to MAX_PER matrices, and in a small
+    batch the kernel takes fewer tiles than the table says (1 / 4096 of the
+    batch's, 1 / 2048 up to n = 16), so larger entries would be the same
+    launch."""
     mpw = 16 if (layout == 1 and n <= RAGGED_QUAD_MAX_N) else 4
+    tiles = -(-batch // mpw)
+    limit = max(1, tiles // (2048 if n <= 16 else 4096))
+    return [g for g in (1, 2, 4, 8, 16) if mpw * g <= MAX_PER and g <= limit]
+
+
+def tune_grab(n: int, layout: int, batch: int, stream: Stream, reps: int = 20) -> tuple[int, dict]:
+    """Ragged path: wave tiles per work item for one n under `layout`.  If the
+    batch is too small for the installed value to be tried and the largest one
+    tried wins, the installed one stays."""
     a = uniform_matrices(2000 + n, batch, n).reshape(-1)
     ns = np.full(batch, n, np.int32)
     offs = np.arange(batch, dtype=np.int64) * (n * n)
@@ -134,9 +147,7 @@ def tune_grab(n: int, layout: int, batch: int, stream: Stream, reps: int = 20) -
     base_l, base_g = api.tuning_get()
     times = {}
     try:
-        for grab in (1, 2, 4, 8, 16):
-            if mpw * grab > MAX_PER:
-                continue
+        for grab in grab_candidates(n, layout, batch):
             g = base_g.copy()
             g[n] = grab
             api.tuning_set(base_l, g)
@@ -156,10 +167,10 @@ def tune_grab(n: int, layout: int, batch: int, stream: Stream, reps: int = 20) -
         for b in (src, work, O, NS, PO, P):
             b.close()
     best = min(times, key=times.get)
-    return best, times
+    return (max(best, int(base_g[n])) if best == max(times) else best), times
 
 
-def autotune(sizes=range(1, 33), plain_batch: int = 262144, ragged_batch: int = 131072, log=None) -> dict:
+def autotune(sizes=range(1, 33), plain_batch: int = 262144, ragged_batch: int = 262144, log=None) -> dict:
     stream = Stream()
     layout, grab = api.tuning_get()
     layout = layout.copy()
@@ -272,7 +283,7 @@ def main(argv=None) -> int:
     ap.add_argument("--out", default="tuning.json")
     ap.add_argument("--sizes", default="1-32")
     ap.add_argument("--plain-batch", type=int, default=262144)
-    ap.add_argument("--ragged-batch", type=int, default=131072)
+    ap.add_argument("--ragged-batch", type=int, default=262144)
     ap.add_argument("--objective", choices=["class", "mix"], default="class",
                     help="class: each n timed alone (plain layout, ragged grab); mix: the ragged table "
                          "tuned on the mixed batch (--mix-batch matrices, n ~ U{2..32})")

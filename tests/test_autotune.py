@@ -49,3 +49,17 @@ def test_apply_table_with_padding(tmp_path):
     finally:
         api.lds_pad_set(pad)
         api.tuning_set(layout, grab)
+
+
+def test_grab_candidates_are_distinct_launches():
+    """Only work-item sizes that the kernel would not clamp to the same launch
+    are timed; the default batch reaches all of them."""
+    from matrixinversion_amd import autotune
+
+    assert autotune.grab_candidates(32, 0, 262144) == [1, 2, 4, 8, 16]
+    assert autotune.grab_candidates(32, 0, 131072) == [1, 2, 4, 8]  # 32,768 tiles / 4096
+    assert autotune.grab_candidates(13, 0, 131072) == [1, 2, 4, 8, 16]
+    assert autotune.grab_candidates(12, 1, 262144) == [1, 2, 4]  # 64 matrices are 4 quad tiles
+    assert autotune.grab_candidates(20, 0, 20000) == [1]
+    import inspect
+    assert inspect.signature(autotune.autotune).parameters["ragged_batch"].default == 262144
