@@ -106,8 +106,8 @@ constexpr int kRaggedLdsFloats = cmax<Geo<32, 16, 1>::LDS_FLOATS, Geo<kRaggedQua
 
 // Matrices start at any float offset, so global accesses are f32x4u.
 
-// Slot offsets of one descriptor, one slot per lane (lanes 0..15; lanes past
-// the descriptor's count repeat slot 0): matrix offset and pivot offset.
+// Slot offsets of one descriptor, one slot per lane (lanes past the
+// descriptor's count repeat slot 0): matrix offset and pivot offset.
 struct RaggedSlots {
   uint32_t so_lo, so_hi, po_lo, po_hi;
 };

@@ -297,8 +297,8 @@ constexpr int kPivGiven = -1;
 // registers allow); keeping the whole tile in registers through the
 // factorisation instead exceeds 256 VGPRs and spills.
 // Against copy + inversion + a refinement pass with every matrix padded to
-// 32 x 32 (300k matrices): n = 12 0.131 ms instead of 0.71, n = 16 0.175, n = 8
-// 0.045.  Bound at n = 12 by the matrix cores' 288 cycles per matrix (35 us)
+// 32 x 32 (300k matrices): n = 12 0.121 ms instead of 0.71; n = 16 0.19, n = 8
+// 0.047.  Bound at n = 12 by the matrix cores' 288 cycles per matrix (35 us)
 // on top of the plain inversion's 54 us, and the chain of each step.
 template <int N, int L, int PIV>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void lu_refined_kernel(

@@ -2,7 +2,7 @@
 //
 // A plan owns the workspace of the device-side planning kernels; enqueueing
 // a batch on a plan allocates nothing and synchronises nothing, so the whole
-// sequence (hist, scan, scatter, invert) can be captured in a hipGraph
+// sequence (at most hist, scan, scatter, invert) can be captured in a hipGraph
 // once and replayed.  lu_batched_inverse_ragged keeps one plan per host
 // thread and grows it when a larger batch arrives.
 #include <hip/hip_runtime.h>
@@ -282,17 +282,17 @@ void plan_release(lub_ragged_plan* p) {
 
 unsigned plan_blocks(int64_t batch) { return static_cast<unsigned>(lub::RaggedWs::blocks(batch)); }
 
-// Matrices per descriptor of class n under tuning `rt` (the scan kernel
-// computes the same).
+// Matrices per descriptor of class n under tuning `rt`, before the device
+// bounds them by the batch's tiles (ragged_grab_limit).
 int ragged_per(const lub::RaggedTuning& rt, int n) {
   const int layout = (rt.layout[n] == 1 && n <= lub::kRaggedQuadMaxN) ? 1 : 0;
   const int mpw = lub::ragged_mpw(n, layout);
   return mpw * std::min(std::max(1, int(rt.grab[n])), lub::kRaggedMaxPer / mpw);
 }
 
-// Grid of the inversion kernel: by default at least the descriptor count
-// (ceil(batch / smallest matrices-per-descriptor) + 32 bounds it), so each
-// workgroup does one descriptor; or ragged_persistent_grid.
+// Grid of the inversion kernel: by default about the descriptor count or
+// above it, so that a workgroup does one descriptor (it strides where the
+// grid is smaller); or ragged_persistent_grid.
 int64_t ragged_grid(int cus, const lub::RaggedTuning& rt, int64_t batch) {
   if (const int64_t persistent = lub::ragged_persistent_grid(cus); persistent > 0) return persistent;
   int min_per = lub::kRaggedMaxPer, min_mpw = lub::kRaggedMaxPer;
@@ -321,7 +321,8 @@ int check_ragged_args(float* A, const int64_t* offsets, const int* ns, int* piv,
   return -1;  // proceed
 }
 
-// The four launches of one ragged batch on `stream`, with the planning
+// The launches of one ragged batch (one without a plan, two with the
+// one-workgroup plan, else four) on `stream`, with the planning
 // workspace at `ws` (lub::RaggedWs layout for `capacity` matrices, batch <=
 // capacity, arguments already checked).  No allocation, no synchronisation.
 int enqueue_ragged(char* ws, int64_t capacity, int cus, float* A, const int64_t* offsets, const int* ns, int* piv,
