@@ -202,10 +202,11 @@ int lu_batched_inverse_refined(const float* A, float* X, int* piv, int n, int64_
  * admission budget) and stay resident until released.  Queued requests of
  * one pivot rule are coalesced into one ragged batch whenever one of the
  * server's launch slots (three, each a stream and a ragged plan) is free, so
- * up to three batches -- of one rule or of several -- run at once.  A request
- * that arrives while a large batch runs starts without waiting for it; behind
- * a short batch of its rule (up to 32,768 matrices) it waits for the end of
- * that, or until as many matrices are queued, and runs with all that came.
+ * up to three batches -- of one rule or of several -- run at once, and a
+ * request that arrives while a batch runs starts without waiting for it.  Only
+ * in a rush (four requests of a rule within 0.2 ms) does a request wait for the
+ * end of a short batch of its rule (up to 32,768 matrices), or until as many
+ * matrices are queued, and runs with all that came.
  * Everything the server uses is allocated by lu_server_create.
  * A result is bit-identical to inverting the same matrices alone.
  * One host thread drives a server; no call blocks except destroy. */

@@ -26,8 +26,9 @@
 //             no plan (up to 2,048 matrices) reads its slot entries from the
 //             pinned staging ring; a larger one gets them in one copy per
 //             array first.  Batches on different slots -- of one rule or of
-//             several -- run concurrently; only behind a short batch of its
-//             own rule does a request wait, and gather with others (kGather).
+//             several -- run concurrently; only in a rush of requests does one
+//             wait behind a short batch of its rule, and gather with
+//             others (kGather).
 //   poll      the tickets finished since the last poll, in completion order.
 //   query     state, device result pointers and end-to-end latency (host clock,
 //             submit to the progress call that saw the batch complete).
@@ -56,17 +57,22 @@ constexpr int kRules = 5;                 // LUB_PIVOT_NONE .. LUB_PIVOT_GEPP
 constexpr int kSlots = 3;                 // batches in flight at once (+ the copy stream = 4 streams)
 constexpr int64_t kAlign = 256;           // request blocks start on 256-byte boundaries
 
-// While a batch of at most kGather matrices (8,192 row tiles, one filling of
-// the chip: about 0.1 ms) of a rule runs, further requests of the rule gather
-// until it is done or kGather matrices wait.  A launch (event, wait, launch,
-// event) costs the host some 20 us, a batch of a few requests ends in about
-// as much, so without this a burst becomes one launch per request and is bound
-// by them.  First-max, us per burst / batches: 64 requests of 1,000 of n =
-// 24..32 1,268 / 8 with, 2,570 / 64 without; 64 of 64 of n = 4..32 1,388 / 18
-// and 2,512 / 64; 32 of 2,000 726 / 5 and 1,318 / 32.  Limits of 2,048 and
-// 16,384 leave larger requests behind (64 of 2,000: 1,981 and 1,629 against
-// 1,370).  A Poisson stream of 16,000 requests/s pays for it in its median
-// (0.056-0.060 -> 0.064-0.072 ms), one of 64,000 gains (0.16 -> 0.135).
+// Requests of a rule that come fast -- this one and the kPress before it within
+// kPressTime -- and find a batch of at most kGather matrices of the rule running
+// (8,192 row tiles, one filling of the chip: about 0.1 ms) gather until it is
+// done or kGather matrices wait.  A launch (event, wait, launch, event) costs
+// the host some 20 us and a batch of a few requests ends in about as much, so
+// without this a burst becomes one launch per request and is bound by them.
+// First-max, us per burst / batches: 64 requests of 1,000 of n = 24..32
+// 1,320 / 10 with, 2,450 / 64 without; 64 of 64 of n = 4..32 1,440 / 20 and
+// 2,400 / 64; 32 of 2,000 790 / 7 and 1,300 / 32.  Limits of 2,048 and 16,384
+// for kGather leave larger requests behind (64 of 2,000: 1,980 and 1,630
+// against 1,370).  Gathering at any pace saves bursts another 5 % and costs a
+// Poisson stream of 16,000 requests/s 12 % of its median (0.061 -> 0.070 ms);
+// at this pace (15,000/s of one rule) it is 0.064, with the same mean and a
+// shorter tail, and at 64,000 requests/s 0.134 instead of 0.177.
+constexpr int kPress = 3;
+constexpr std::chrono::microseconds kPressTime{200};
 constexpr int64_t kGather = 32768;
 
 int64_t round_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
@@ -120,6 +126,8 @@ struct Rule {
   std::deque<uint64_t> queued;    // tickets in submission order
   std::deque<RingRun> runs;       // launched batches not yet reclaimed
   int inflight = 0;               // batches of this rule running now
+  Clock::time_point came[kPress + 1] = {};  // ring: when the last requests came
+  int64_t ncame = 0;
 };
 
 }  // namespace
@@ -252,6 +260,9 @@ int retire(lub_server* s, int* completed) {
 // Whether `rule`'s queued requests wait for more (see kGather).
 bool gathering(lub_server* s, int rule) {
   const Rule& r = s->rules[rule];
+  if (r.ncame <= kPress) return false;
+  // of the ring's kPress + 1 times, the next to be overwritten is the oldest
+  if (r.came[(r.ncame - 1) % (kPress + 1)] - r.came[r.ncame % (kPress + 1)] > kPressTime) return false;
   if (r.head - find(s, r.queued.front())->slot >= std::min(kGather, s->max_batch)) return false;
   for (const Slot& sl : s->slots)
     if (sl.busy && sl.rule == rule && sl.count <= kGather) return true;
@@ -410,6 +421,7 @@ int lu_server_submit(lub_server* s, const float* src, const int* ns, int count, 
   rq.floats = floats;
   rq.slot = slot;
   rq.t_submit = Clock::now();
+  r.came[r.ncame++ % (kPress + 1)] = rq.t_submit;
   s->head = new_head;
   r.head = slot + count;
   r.queued.push_back(rq.ticket);
